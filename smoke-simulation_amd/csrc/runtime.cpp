@@ -248,6 +248,22 @@ smoke_status ensure_vort(smoke_sim* s)
     return SMOKE_OK;
 }
 
+// Allocates the reference projection's second velocity set (once per
+// simulation, before a step or a capture).  Its launches write every entry
+// they later read.
+void ensure_sweep_fields(smoke_sim* s)
+{
+    if (s->prm.projection != SMOKE_PROJ_REFERENCE || s->sweep_mem || s->sweep_refused) return;
+    const size_t field = align256((size_t)s->g.elems * sizeof(float));
+    if (hipMalloc((void**)&s->sweep_mem, 3 * field) != hipSuccess) {
+        smk::forget_last_error();  // the launches' checks must not find it
+        s->sweep_mem = nullptr;
+        s->sweep_refused = true;
+        return;
+    }
+    for (int k = 0; k < 3; ++k) s->sweep_vel[k] = reinterpret_cast<float*>(s->sweep_mem + k * field);
+}
+
 // Allocates the step-norms records (once per simulation): the reduction's
 // scratch, then the public record it publishes.
 size_t norms_bytes() { return align256(smk::norms_scratch_bytes()) + sizeof(smoke_step_norms); }
@@ -433,14 +449,21 @@ hipError_t stage_project(smoke_sim* s, long long* launches)
             *launches += 1;
         }
         if ((e = sweep_mark(s, 0, 0)) != hipSuccess) return e;
-        for (int it = 0; it < p.iterations; ++it)
-            for (int o = 0; o < 2; ++o) {
-                e = smk::project_reference_half(g, s->u[n], s->v[n], s->w[n], s->flags, o,
+        int n_launches = 2 * p.iterations;
+        if (s->sweep_mem && p.iterations >= 2) {
+            float* const vel[3] = {s->u[n], s->v[n], s->w[n]};
+            e = smk::project_reference_sweeps(g, vel, s->sweep_vel, s->flags, 2 * p.iterations,
+                                              p.sor_omega, s->stream, &n_launches);
+            if (e != hipSuccess) return e;
+        } else {
+            for (int k = 0; k < n_launches; ++k) {
+                e = smk::project_reference_half(g, s->u[n], s->v[n], s->w[n], s->flags, k & 1,
                                                 p.sor_omega, s->stream);
                 if (e != hipSuccess) return e;
-                *launches += 1;
             }
-        return sweep_mark(s, 1, 2LL * p.iterations);
+        }
+        *launches += n_launches;
+        return sweep_mark(s, 1, n_launches);
     }
     e = smk::with_fields(s, [&](auto, auto u, auto v, auto w) {
         return smk::divergence(g, u[n], v[n], w[n], s->flags, s->d, s->stream);
@@ -647,6 +670,7 @@ smoke_status step_locked(smoke_sim* s, float dt)
 {
     SMOKE_REFUSE_IN_BATCH(s, "step");
     if (!std::isfinite(dt)) return fail(SMOKE_ERR_INVALID, "step: dt must be finite");
+    ensure_sweep_fields(s);
     if (s->graph_on && !s->timing && !s->norms_on) return step_graph(s, dt);
     smoke_sim::StepEvents se{};
     if (s->timing) {
@@ -859,6 +883,7 @@ void smoke_destroy(smoke_sim* s)
     if (s->copy_stream) (void)hipStreamDestroy(s->copy_stream);
     if (s->refine_mem) (void)hipFree(s->refine_mem);
     if (s->vort_mem) (void)hipFree(s->vort_mem);
+    if (s->sweep_mem) (void)hipFree(s->sweep_mem);
     if (s->owner) (void)hipFree(s->owner);
     if (s->norms_mem) (void)hipFree(s->norms_mem);
     if (s->arena) (void)hipFree(s->arena);
@@ -1449,6 +1474,7 @@ smoke_status smoke_run_stage(smoke_sim* s, int stage, float dt)
     SMOKE_REFUSE_IN_BATCH(s, "run_stage");
     s->norms_step = -1;
     s->last_dt = dt;
+    ensure_sweep_fields(s);
     long long launches = 0;
     hipError_t e = run_stage(s, stage, dt, &launches);
     if (e != hipSuccess) return fail(SMOKE_ERR_HIP, "run_stage %d: %s", stage, hipGetErrorString(e));

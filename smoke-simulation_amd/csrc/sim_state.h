@@ -64,6 +64,12 @@ struct smoke_sim {
     // above 0).
     char* vort_mem = nullptr;
     smk::VortBufs vb{};
+    // Second set of velocity fields of the reference projection's half-sweeps
+    // (allocated before the first step that uses them; without memory for
+    // them, sweep_refused, the half-sweeps run in place, one per launch).
+    char* sweep_mem = nullptr;
+    bool sweep_refused = false;
+    float* sweep_vel[3] = {nullptr, nullptr, nullptr};
     // Moving-obstacle boundary condition: per-cell owner bytes (allocated
     // when obstacle_velocity is first set; built with the mask).
     uint8_t* owner = nullptr;

@@ -28,6 +28,8 @@ struct Grid {
     }
 };
 
+constexpr int kCUs = 256;  // compute units of an MI355X
+
 // Thread block of the per-cell kernels (64 x 4: one wave64 per row segment).
 constexpr int kBlockX = 64;
 constexpr int kBlockY = 4;
@@ -245,9 +247,18 @@ struct VortBufs {
 hipError_t vorticity(const Grid& g, float* u, float* v, float* w, const uint8_t* flags,
                      const VortBufs& b, float eps, float dt, hipStream_t st);
 
+// Clears the thread's last HIP error (left by a call whose failure was handled).
+void forget_last_error();
+
 // Projection.
 hipError_t project_reference_half(const Grid& g, float* u, float* v, float* w,
                                   const uint8_t* flags, int colour, double omega, hipStream_t st);
+// `sweeps` half-sweeps (an even number, at least 2) in a few launches
+// (redblack.h), alternating between the fields a (u, v, w) and b (three
+// scratch fields of the same layout); the result is in a.
+hipError_t project_reference_sweeps(const Grid& g, float* const (&a)[3], float* const (&b)[3],
+                                    const uint8_t* flags, int sweeps, double omega, hipStream_t st,
+                                    int* launches);
 hipError_t divergence(const Grid& g, const float* u, const float* v, const float* w,
                       const uint8_t* flags, float* d, hipStream_t st);
 hipError_t jacobi_sweep(const Grid& g, const float* pin, float* pout, const float* d,

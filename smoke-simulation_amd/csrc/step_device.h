@@ -24,6 +24,20 @@ namespace dev {
 constexpr int BX = kBlockX;
 constexpr int BY = kBlockY;
 
+// Tile order of the tiled kernels.  Workgroup b runs on XCD b % 8 (8 XCDs,
+// each with its own L2): the tiles are renumbered so that each XCD gets one
+// contiguous run of tiles (x fastest), and tiles that share halo cells run on
+// the same L2 at the same time.  The renumbering is a permutation (the tail
+// beyond a multiple of 8 keeps its index).
+__device__ __forceinline__ int xcd_tile_order()
+{
+    const int nbx = (int)gridDim.x, nby = (int)gridDim.y;
+    const int nb = nbx * nby * (int)gridDim.z;
+    const int b = (int)blockIdx.x + nbx * ((int)blockIdx.y + nby * (int)blockIdx.z);
+    const int full = nb & ~7;
+    return (b < full) ? (b & 7) * (full >> 3) + (b >> 3) : b;
+}
+
 // Sphere membership as fillSmoke/fillObstacle test it
 // (smokeSimulation.cu:265, :304): integer cell index, float centre, squares
 // and sums in float, strict comparison with r*r.

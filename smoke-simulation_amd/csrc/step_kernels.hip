@@ -13,6 +13,7 @@
 // FP32 mode.
 #include <algorithm>
 
+#include "redblack.h"
 #include "step_device.h"
 
 namespace smk {
@@ -344,20 +345,6 @@ __global__ void k_jacobi(Grid g, const float* __restrict__ pin, float* __restric
                    blockIdx.y * BY + threadIdx.y + 1, blockIdx.z + 1);
 }
 
-// Tile order of the tiled kernels.  Workgroup b runs on XCD b % 8 (8 XCDs,
-// each with its own L2): the tiles are renumbered so that each XCD gets one
-// contiguous run of tiles (x fastest), and tiles that share halo cells run on
-// the same L2 at the same time.  The renumbering is a permutation (the tail
-// beyond a multiple of 8 keeps its index).
-__device__ __forceinline__ int xcd_tile_order()
-{
-    const int nbx = (int)gridDim.x, nby = (int)gridDim.y;
-    const int nb = nbx * nby * (int)gridDim.z;
-    const int b = (int)blockIdx.x + nbx * ((int)blockIdx.y + nby * (int)blockIdx.z);
-    const int full = nb & ~7;
-    return (b < full) ? (b & 7) * (full >> 3) + (b >> 3) : b;
-}
-
 // T fused Jacobi sweeps, one TX x TY tile per block of TX x (TY / R) threads
 // (dev::jacobi_fused_tile).  One row per thread: at most 64 VGPRs, two
 // 1024-thread blocks per CU; two rows per thread: at most 128 VGPRs.
@@ -368,7 +355,7 @@ __global__ __launch_bounds__(TX * TY / R, 8 / R) void k_jacobi_fused(
 {
     __shared__ dev::FusedLds<TX, TY, T> sh;
     const int nbx = (int)gridDim.x, nby = (int)gridDim.y;
-    const int L = xcd_tile_order();
+    const int L = dev::xcd_tile_order();
     dev::jacobi_fused_tile<TX, TY, T, DAMPED, R>(g, pin, pout, d, flags, zc, zero_in, omega,
                                                  L % nbx, (L / nbx) % nby, L / (nbx * nby), sh);
 }
@@ -452,7 +439,7 @@ __global__ __launch_bounds__(BX * BY) void k_advect_velocity(
 {
     __shared__ dev::AdvRing<BX, BY, 4, 3> ring;
     const int nbx = (int)gridDim.x, nby = (int)gridDim.y;
-    const int L = xcd_tile_order();
+    const int L = dev::xcd_tile_order();
     dev::advect_velocity_march<BY, kAdvZC>(g, u0, v0, w0, u1, v1, w1, flags, dt,
                                            1 + BX * (L % nbx), 1 + BY * ((L / nbx) % nby),
                                            1 + kAdvZC * (L / (nbx * nby)), ring);
@@ -467,7 +454,7 @@ __global__ __launch_bounds__(BX * BY) void k_advect_density(
 {
     __shared__ dev::AdvRing<BX, BY, 4, 1, 2> ring;
     const int nbx = (int)gridDim.x, nby = (int)gridDim.y;
-    const int L = xcd_tile_order();
+    const int L = dev::xcd_tile_order();
     dev::advect_density_march<BY, kAdvZC>(g, r0, r1, u, v, w, flags, dt, BX * (L % nbx),
                                           1 + BY * ((L / nbx) % nby),
                                           1 + kAdvZC * (L / (nbx * nby)), ring);
@@ -668,6 +655,8 @@ hipError_t vorticity(const Grid& g, float* u, float* v, float* w, const uint8_t*
     return launch_vorticity(g, u, v, w, flags, b, eps, dt, st);
 }
 
+void forget_last_error() { (void)hipGetLastError(); }
+
 hipError_t project_reference_half(const Grid& g, float* u, float* v, float* w,
                                   const uint8_t* flags, int colour, double omega, hipStream_t st)
 {
@@ -678,6 +667,46 @@ hipError_t project_reference_half(const Grid& g, float* u, float* v, float* w,
     hipLaunchKernelGGL(k_project_ref_half, grid, dim3(BX, BY), 0, st, g, u, v, w, flags, colour,
                        omega, pairs);
     return hipGetLastError();
+}
+
+hipError_t project_reference_sweeps(const Grid& g, float* const (&a)[3], float* const (&b)[3],
+                                    const uint8_t* flags, int sweeps, double omega, hipStream_t st,
+                                    int* launches)
+{
+    // At most one box per CU: boxes (redblack.h has both sides).  Else columns:
+    // 6 half-sweeps per launch where the two sets of faces and the flags
+    // approach the 256 MB memory-side cache (a launch is then bound by memory
+    // and fewer passes pay for the larger halo), 4 where they do not.  us per
+    // half-sweep with 4 / 6: 160^3 (125 MB) 8.1 / 8.4, 192x180x188 (191 MB)
+    // 10.7 / 10.2, 224x200x210 (271 MB) 18.0 / 14.1, 256x240x248 29.8 / 22.4.
+    constexpr int IX = 24, IY = 10, IZ = 10;
+    const dim3 boxes((unsigned)((g.nx + IX - 1) / IX), (unsigned)((g.ny + IY - 1) / IY),
+                     (unsigned)((g.nz + IZ - 1) / IZ));
+    const bool boxed = (long long)boxes.x * boxes.y * boxes.z <= kCUs;
+    const bool large = (long long)g.elems * 25 > (150LL << 20);
+    const int H = !boxed && large ? 6 : 4;
+    // An even number of launches, so that the last one writes a again.
+    const int n = 2 * ((sweeps + 2 * H - 1) / (2 * H));
+    *launches = 0;
+    for (int l = 0, done = 0; l < n; ++l) {
+        const int m = sweeps / n + (l < sweeps % n ? 1 : 0), colour = done & 1;
+        float* const* in = l & 1 ? b : a;
+        float* const* out = l & 1 ? a : b;
+        const FaceSets f = {in[0], in[1], in[2], out[0], out[1], out[2]};
+        hipError_t e;
+        if (boxed) {
+            hipLaunchKernelGGL((k_ref_faces_box<IX, IY, IZ, 4>), boxes, dim3(kBoxThreads), 0, st, g,
+                               f.ui, f.vi, f.wi, f.uo, f.vo, f.wo, flags, colour, m, omega);
+            e = hipGetLastError();
+        } else {
+            e = large ? launch_faces_march<6>(g, f, flags, colour, m, omega, st)
+                      : launch_faces_march<4>(g, f, flags, colour, m, omega, st);
+        }
+        if (e != hipSuccess) return e;
+        done += m;
+        ++*launches;
+    }
+    return hipSuccess;
 }
 
 template <typename T>
