@@ -183,9 +183,10 @@ smoke_status smoke_get_params(const smoke_sim* sim, smoke_params* out);
 
 /* Launch plan of the fused Jacobi sweeps (SMOKE_PROJ_JACOBI): how many sweeps
  * one launch fuses (1..6), the thread-block tile and the z-chunk length.
- * Every plan gives bit-identical results; only the speed differs.  No
- * reference counterpart (the reference launches one kernel per half-sweep,
- * smokeSimulation.cu:797-801). */
+ * Every plan gives bit-identical results; only the speed differs.  A
+ * simulation whose plan was never set (get returns the defaults below) runs
+ * one fitted to its grid.  No reference counterpart (the reference launches
+ * one kernel per half-sweep, smokeSimulation.cu:797-801). */
 /* Tiles 64x32 and 32x64 give each thread two rows of its column (fewer halo
  * cells per written cell, one 1024-thread block per CU instead of two). */
 typedef enum smoke_tile {

@@ -371,10 +371,11 @@ hipError_t enqueue_refined(smoke_sim* s, long long* launches, long long* sweep_l
     const smoke_params& p = s->prm;
     const smk::RefineBufs& b = s->rb;
     const int R = (p.iterations + p.inner_sweeps - 1) / p.inner_sweeps;
-    int T = s->plan.sweeps_per_launch;
+    const smk::JacobiPlan plan = s->plan_set ? s->plan : smk::fitted_plan(g, true);
+    int T = plan.sweeps_per_launch;
     if (T < 2 || T > 6 || (T & 1)) T = 4;
-    const int two_rows = (s->plan.tile == smk::JacobiPlan::TILE_64x32 ||
-                          s->plan.tile == smk::JacobiPlan::TILE_32x64) ? 1 : 0;
+    const int two_rows = (plan.tile == smk::JacobiPlan::TILE_64x32 ||
+                          plan.tile == smk::JacobiPlan::TILE_32x64) ? 1 : 0;
     hipError_t e = smk::refine_norm0(g, s->d, s->flags, b, p.tolerance, s->stream);
     if (e != hipSuccess) return e;
     *launches += 2;
@@ -386,7 +387,7 @@ hipError_t enqueue_refined(smoke_sim* s, long long* launches, long long* sweep_l
             const int t = std::min(left, T);
             const int eout = first ? 0 : 1 - ein;
             e = smk::refine_sweeps(g, b, r == 0 ? s->d : b.q, s->flags, first ? 1 : 0, ein, eout, t,
-                                   s->plan.zc, two_rows, s->stream);
+                                   plan.zc, two_rows, s->stream);
             if (e != hipSuccess) return e;
             ein = eout;
             first = false;
@@ -492,7 +493,8 @@ hipError_t stage_project(smoke_sim* s, long long* launches)
         }
         if ((e = sweep_mark(s, 0, 0)) != hipSuccess) return e;
         long long sweep_launches = 0;
-        e = enqueue_jacobi(s, s->plan, p.iterations, zero_in, &sweep_launches);
+        e = enqueue_jacobi(s, s->plan_set ? s->plan : smk::fitted_plan(g, false), p.iterations, zero_in,
+                           &sweep_launches);
         if (e != hipSuccess) return e;
         *launches += sweep_launches;
         if ((e = sweep_mark(s, 1, sweep_launches)) != hipSuccess) return e;
@@ -1241,6 +1243,9 @@ smoke_status smoke_restore(smoke_sim* s, const void* host, size_t bytes)
     s->plan.sweeps_per_launch = h.plan[0];
     s->plan.tile = h.plan[1];
     s->plan.zc = h.plan[2];
+    const smk::JacobiPlan unset;
+    s->plan_set = s->plan.sweeps_per_launch != unset.sweeps_per_launch || s->plan.tile != unset.tile ||
+                  s->plan.zc != unset.zc;
     s->version += 1;
     s->mask_dirty = true;  // flags (and the refined solver's inverse) follow the restored masks
     HIP_TRY(refresh_mask(s, nullptr));
@@ -1274,6 +1279,7 @@ smoke_status smoke_set_jacobi_plan(smoke_sim* s, const smoke_jacobi_plan* plan)
     s->plan.sweeps_per_launch = plan->sweeps_per_launch;
     s->plan.tile = plan->tile;
     s->plan.zc = plan->zc;
+    s->plan_set = true;
     s->version += 1;
     return SMOKE_OK;
 }
@@ -1322,6 +1328,7 @@ smoke_status smoke_autotune(smoke_sim* s, smoke_jacobi_plan* chosen, double* ms_
     const bool refined = s->prm.projection == SMOKE_PROJ_REFINED;
     const int pcur0 = s->pcur;
     const smk::JacobiPlan plan0 = s->plan;
+    const bool plan_set0 = s->plan_set;
     const long long fp16_sweeps =
         (long long)((s->prm.iterations + s->prm.inner_sweeps - 1) / s->prm.inner_sweeps) *
         s->prm.inner_sweeps;
@@ -1342,7 +1349,18 @@ smoke_status smoke_autotune(smoke_sim* s, smoke_jacobi_plan* chosen, double* ms_
             if (e != hipSuccess) break;
             if (refined && tile != smk::JacobiPlan::TILE_32x32 && tile != smk::JacobiPlan::TILE_64x32)
                 continue;  // the refined sweeps have one tile per row count
-            for (int zc : zcs) {
+            // And the chunks that give one and two workgroups per CU.
+            std::vector<int> lengths = zcs;
+            const int w = refined ? 64 : smk::tile_width(tile), h = refined ? (tile == tiles[0] ? 32 : 64)
+                                                                            : smk::tile_height(tile);
+            const int columns = ((refined ? s->g.px : s->g.nx - 2) + w - 2 * t - 1) / (w - 2 * t) *
+                                ((s->g.ny - 2 + h - 2 * t - 1) / (h - 2 * t));
+            for (int per_cu = 1; per_cu <= 2; ++per_cu) {
+                const int chunks = std::max(1, per_cu * smk::kCUs / columns);
+                const int zc = std::max(1, (s->g.nz - 2 + chunks - 1) / chunks);
+                if (std::find(lengths.begin(), lengths.end(), zc) == lengths.end()) lengths.push_back(zc);
+            }
+            for (int zc : lengths) {
                 smk::JacobiPlan cand;
                 cand.sweeps_per_launch = t;
                 cand.tile = tile;
@@ -1351,6 +1369,7 @@ smoke_status smoke_autotune(smoke_sim* s, smoke_jacobi_plan* chosen, double* ms_
                 auto run = [&]() {
                     if (!refined) return enqueue_jacobi(s, cand, K, false, &n);
                     s->plan = cand;
+                    s->plan_set = true;
                     const hipError_t r = enqueue_refined(s, &n, &n2);
                     s->pcur = pcur0;
                     return r;
@@ -1372,6 +1391,7 @@ smoke_status smoke_autotune(smoke_sim* s, smoke_jacobi_plan* chosen, double* ms_
         }
     }
     s->plan = plan0;
+    s->plan_set = plan_set0;
     s->pcur = pcur0;
     // The sweeps ran on whatever right-hand side the buffer held: start the
     // next warm start from zero.
@@ -1381,6 +1401,7 @@ smoke_status smoke_autotune(smoke_sim* s, smoke_jacobi_plan* chosen, double* ms_
     cleanup();
     if (e != hipSuccess) return fail(SMOKE_ERR_HIP, "autotune: %s", hipGetErrorString(e));
     s->plan = best;
+    s->plan_set = true;
     s->version += 1;
     if (chosen) {
         chosen->sweeps_per_launch = best.sweeps_per_launch;

@@ -93,6 +93,9 @@ struct smoke_sim {
     int pcur = 0;  // P buffer holding the latest pressure
     bool mask_dirty = true;
     smk::JacobiPlan plan;  // launch plan of the fused Jacobi sweeps
+    // Set by a caller, the autotuner or a snapshot; a plan that was not gives
+    // way to the one fitted to the grid (same bits).
+    bool plan_set = false;
     smoke_batch* batch = nullptr;         // batch this simulation belongs to
     hipStream_t batch_stream = nullptr;   // that batch's stream
     long long steps_enqueued = 0;

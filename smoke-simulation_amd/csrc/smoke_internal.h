@@ -108,6 +108,40 @@ inline int tile_height(int tile)
     return tile == JacobiPlan::TILE_64x16 ? 16 : (tile == JacobiPlan::TILE_32x64 ? 64 : 32);
 }
 
+// Planes per workgroup, at most `most`, for launches of `tiles` columns over
+// `planes` planes, a workgroup marching its planes and `fill` more, the sum
+// rounded up to `unroll`: the fewest steps of the busiest CU, by a model of
+// the step time (us) with one workgroup on a CU (`one`) and with as many as
+// fit (`full`, `resident` of them).  Also the modelled time of the launch.
+struct ChunkModel {
+    int fill, unroll, resident;
+    double one, full;
+};
+inline int fit_chunk(const ChunkModel& m, int tiles, int planes, int most, double* us)
+{
+    int best = most < planes ? most : planes;
+    double best_us = -1.0;
+    for (int chunks = 1; chunks <= planes; ++chunks) {
+        const int zc = (planes + chunks - 1) / chunks;
+        if (zc > most) continue;
+        const long long blocks = (long long)tiles * ((planes + zc - 1) / zc);
+        const int steps = (zc + m.fill + m.unroll - 1) / m.unroll * m.unroll;
+        const long long per_round = (long long)kCUs * m.resident;
+        const double t = blocks <= kCUs ? steps * m.one
+                                        : steps * m.full * (double)((blocks + per_round - 1) / per_round);
+        if (best_us < 0.0 || t < best_us) {
+            best_us = t;
+            best = zc;
+        }
+        if (blocks > 4 * per_round) break;  // smaller chunks only add fill
+    }
+    *us = best_us;
+    return best;
+}
+// The plan of a simulation whose plan was never set (step_kernels.hip), for
+// the Jacobi sweeps and for the refined solve's FP16 sweeps.
+JacobiPlan fitted_plan(const Grid& g, bool refined);
+
 // ------------------------------------------------------------- batching
 
 // One simulation as the batched kernels see it (device memory).  `now` and

@@ -765,6 +765,45 @@ static hipError_t launch_fused_t(const Grid& g, const float* pin, float* pout, c
     }
 }
 
+// A plan that was never set follows the grid: with the plan's own 64 planes per
+// workgroup a small grid occupies a handful of CUs (48x40x57: 4 workgroups,
+// 30.6 us per 4 sweeps; fitted 8.2 us per 5) and a middling one fills the last
+// round of CUs badly (197x131x243: 36.5 us per 4, fitted 30.1 per 5).  Five
+// sweeps per launch, whose loop is unrolled by 6 planes only, were the fastest
+// per sweep at every size measured (48x40x57 to 512^3), in 32x32 tiles (two
+// workgroups per CU) on small grids and 64x32 tiles on large ones.  The step
+// times are measured on full-size tiles of those grids; where the fields
+// outgrow the 256 MB memory-side cache, a launch takes at least the tiles'
+// re-read bytes at 4.9 TB/s.
+JacobiPlan fitted_plan(const Grid& g, bool refined)
+{
+    JacobiPlan plan;
+    const int m[3] = {g.nx - 2, g.ny - 2, g.nz - 2};
+    const int most = std::max(1, fused_max_zc(g.plane));
+    auto columns = [&](int w, int h, int ox, int oy) { return (w + ox - 1) / ox * ((h + oy - 1) / oy); };
+    double us = 0.0;
+    if (refined) {
+        // FP16 pairs: 64x32-cell tiles (two per CU) of 4 sweeps, as unset plans had.
+        constexpr int T = 4;
+        const ChunkModel half{2 * T, 15, 2, 0.45, 0.70};
+        plan.zc = fit_chunk(half, columns(g.px, m[1], 64 - 2 * T, 32 - 2 * T), m[2], std::min(64, most), &us);
+        return plan;
+    }
+    constexpr int T = 5;
+    plan.sweeps_per_launch = T;
+    const double cells = (double)m[0] * m[1] * m[2];
+    const double memory = cells * 13.0 > 256e6 ? cells * 13.0 / 4.9e6 : 0.0;  // us, halo apart
+    const ChunkModel one_row{2 * T, 6, 2, 0.42, 0.66}, two_rows{2 * T, 6, 1, 0.72, 0.73};
+    plan.zc = fit_chunk(one_row, columns(m[0], m[1], 32 - 2 * T, 32 - 2 * T), m[2], most, &us);
+    const double one_us = std::max(us, 1.6 * memory);
+    const int zc = fit_chunk(two_rows, columns(m[0], m[1], 64 - 2 * T, 32 - 2 * T), m[2], most, &us);
+    if (std::max(us, 1.27 * memory) < one_us) {
+        plan.tile = JacobiPlan::TILE_64x32;
+        plan.zc = zc;
+    }
+    return plan;
+}
+
 hipError_t jacobi_fused(const Grid& g, const float* pin, float* pout, const float* d,
                         const uint8_t* flags, const JacobiPlan& plan, int sweeps, float omega,
                         int plain, int zero_in, hipStream_t st)
