@@ -16,10 +16,10 @@
 // 13.3 us per launch of 4 half-sweeps (2.3 the launch itself, 5 the loads and
 // stores, 1.4 each half-sweep), 4 x 4.6 us one by one, 16.4 us marched.
 // Larger grids (k_ref_faces_march): a column marched up z re-reads far less
-// halo.  256x240x248, 6 half-sweeps per launch: 134 us against 6 x 85 us; 4
-// per launch: 119 us (memory-bound, 4.8 TB/s); boxes: 306 us per 4.
-// 150x96x121, 4 per launch: 22.5 us against 4 x 11.2 us (6 per launch 35.5,
-// boxes 42 per 4): there FP64 conversions and VALU issue bind.
+// halo.  256x240x248, 5 half-sweeps per launch: 133 us against 5 x 85 us; boxes
+// 306 us per 4.  150x96x121, 4 per launch: 24 us against 4 x 11.2 us (boxes 42
+// per 4): there FP64 conversions and VALU issue bind (2 % of the cells next to
+// a solid), memory at 256.
 #pragma once
 
 #include "step_device.h"
@@ -27,36 +27,51 @@
 namespace smk {
 namespace {
 
-// Relaxes a cell on its six faces f (u low, u high, v low, ...), as
-// k_project_ref_half does, in two parts.
+// The diagonal of a cell by its flags: RN(1 / fluid neighbours) in FP64, one
+// entry per combination of the six neighbour bits.
+struct FaceDiagonal {
+    double inv[64];
+    __device__ __forceinline__ double of(uint32_t c) const { return inv[(c & F_NBRS) >> 1]; }
+    __device__ __forceinline__ void fill(int tid)
+    {
+        if (tid < 64) inv[tid] = tid ? 1.0 / (double)__popc((unsigned)tid) : 0.0;
+    }
+};
+
+// Relaxes an active cell with flags c on its six faces f (u low, u high, v low,
+// ...), as k_project_ref_half does; other cells keep theirs.
 //
-// Cells with six fluid neighbours (nearly all): the divisor is 6 and every face
-// moves.  -dv / 6 is RN(double(-dv) * RN(1/6)): the FP64 product is within
-// 2^-52 of the quotient, and no quotient by 6 comes that near a rounding
-// boundary of FP32 without lying on it exactly (all 2^32 floats compared on
-// the CPU).  Straight-line code for every lane: others subtract +0 and add
-// -0, which leave every face as it was.
-__device__ __forceinline__ void relax_full(bool full, double omega, float (&f)[6])
+// -dv / n is RN(double(-dv) * RN(1/n)): the FP64 product is within 2^-52 of the
+// quotient, and no quotient by n = 1..6 comes that near a rounding boundary of
+// FP32 without lying on it exactly (all 2^32 floats compared on the CPU for 3,
+// 5 and 6; 1, 2 and 4 are exact).  Cells with six fluid neighbours (nearly
+// all) move every face, in straight-line code for every lane: others subtract
+// +0 and add -0, which leave any face as it was.  Next to a solid a face moves
+// by p * 0, a zero of p's sign or NaN, as the reference's product does.
+__device__ __forceinline__ void relax_faces(uint32_t c, double inv, double omega, float (&f)[6])
 {
     const float dv = -f[0] + f[1] + -f[2] + f[3] + -f[4] + f[5];
-    const float q = (float)((double)(-dv) * (1.0 / 6.0));
+    const float q = (float)((double)(-dv) * inv);
     const float p = (float)((double)q * omega);
+    constexpr uint32_t kFull = F_ACTIVE | F_SELF | F_NBRS;
+    const bool full = c == kFull;
     const float sub = full ? p : 0.0f, add = full ? p : -0.0f;
 #pragma unroll
     for (int k = 0; k < 6; k += 2) {
         f[k] = f[k] - sub;
         f[k + 1] = f[k + 1] + add;
     }
-}
-// Cells next to a solid.
-__device__ __forceinline__ void relax_partial(uint32_t c, double omega, float (&f)[6])
-{
-    const float dv = -f[0] + f[1] + -f[2] + f[3] + -f[4] + f[5];
-    const float p = (float)((double)(-dv / (float)__popc(c & F_NBRS)) * omega);
+    if (c >= F_ACTIVE && !full) {
+        const uint32_t on = __float_as_uint(p), off = __float_as_uint(p * 0.0f);
+        auto step = [&](int bit) {
+            const uint32_t m = (uint32_t)((int32_t)(c << (31 - bit)) >> 31);
+            return __uint_as_float((on & m) | (off & ~m));
+        };
 #pragma unroll
-    for (int k = 0; k < 6; k += 2) {
-        f[k] = f[k] - p * (float)((c >> (k + 1)) & 1);
-        f[k + 1] = f[k + 1] + p * (float)((c >> (k + 2)) & 1);
+        for (int k = 0; k < 6; k += 2) {
+            f[k] = f[k] - step(k + 1);
+            f[k + 1] = f[k + 1] + step(k + 2);
+        }
     }
 }
 
@@ -83,7 +98,9 @@ __global__ __launch_bounds__(kBoxThreads) void k_ref_faces_box(
     using S = FaceBox<IX, IY, IZ, H>;
     __shared__ __align__(16) float f[3][2][S::N];
     __shared__ __align__(16) uint16_t fl[S::N];  // the pair's two flags bytes
+    __shared__ FaceDiagonal diag;
     const int tid = (int)threadIdx.x;
+    diag.fill(tid);
     const int nbx = (int)gridDim.x, nby = (int)gridDim.y;
     const int b = dev::xcd_tile_order();
     const int xa = IX * (b % nbx) - H, ya = IY * ((b / nbx) % nby) - H, za = IZ * (b / (nbx * nby)) - H;
@@ -158,8 +175,7 @@ __global__ __launch_bounds__(kBoxThreads) void k_ref_faces_box(
                 float* const v0 = u0 + 2 * S::N;
                 float* const w0 = u0 + 4 * S::N;
                 float face[6] = {u0[0], u1[0], v0[0], v0[S::TP], w0[0], w0[S::ZS]};
-                if ((c & F_NBRS) == F_NBRS) relax_full(true, omega, face);
-                else relax_partial(c & 0xffu, omega, face);
+                relax_faces(c & 0xffu, diag.of(c), omega, face);
                 u0[0] = face[0];
                 u1[0] = face[1];
                 v0[0] = face[2];
@@ -200,8 +216,11 @@ __global__ __launch_bounds__(kBoxThreads) void k_ref_faces_box(
 // there one pair more than H cells goes stale.
 template <int TP, int TY, int H>
 struct FaceColumn {
-    static_assert(H % 2 == 0 && 64 % TP == 0, "whole pairs, whole rows per wave");
+    static_assert(64 % TP == 0, "whole rows per wave");
     static constexpr int IX = 2 * TP - 2 * H - 2, IY = TY - 2 * H;  // owned faces
+    // First owned pair of a row (whole pairs: with an even H the odd rows'
+    // owned pairs start and end one earlier).
+    static __device__ __forceinline__ int first(int skew) { return (H + 2) / 2 - (H % 2 == 0 ? skew : 0); }
     // Planes in flight: k+1 (entering) down to k-2H+1 (leaving), and one more
     // for an even count, so that a slot's colour does not change.
     static constexpr int W = 2 * H + 2;
@@ -222,17 +241,19 @@ __global__ __launch_bounds__(TP * TY) void k_ref_faces_march(
     using S = FaceColumn<TP, TY, H>;
     constexpr int W = S::W, D = 2;  // D planes of prefetch (W % D == 0)
     __shared__ float lv[W * S::SLOT];
+    __shared__ FaceDiagonal diag;
     const int t = (int)threadIdx.x, r = (int)threadIdx.y;
+    diag.fill(t + TP * r);
     const int nbx = (int)gridDim.x, nby = (int)gridDim.y;
     const int b = dev::xcd_tile_order();
-    const int xa = S::IX * (b % nbx) - H - 2, ya = S::IY * ((b / nbx) % nby) - H;
+    const int xa = S::IX * (b % nbx) - (H + 2) / 2 * 2, ya = S::IY * ((b / nbx) % nby) - H;
     const int z0 = zc * (b / (nbx * nby)), z1 = min(z0 + zc, g.nz);
     const int y = ya + r, skew = y & 1, x0 = xa + 2 * t + skew;
     const bool inside = x0 >= 0 && x0 < g.nx && y >= 0 && y < g.ny;
     // Lanes outside the grid read its first cells and have no flags.
     const uint32_t lane = inside ? (uint32_t)g.idx(x0, y, 0) : 0u;
     const uint32_t fmask = inside ? 0xffffu : 0u;
-    const bool owner = inside && t >= H / 2 + 1 - skew && t < TP - H / 2 - skew && r >= H && r < TY - H;
+    const bool owner = inside && t >= S::first(skew) && t < S::first(skew) + S::IX / 2 && r >= H && r < TY - H;
     // LDS index of the y face of the pair's first and second cell in slot 0.
     const int l0 = r * S::ROW + t + (skew ? TP + 1 : 0);
     const int l1 = r * S::ROW + t + (skew ? 1 : TP + 1);
@@ -293,9 +314,7 @@ __global__ __launch_bounds__(TP * TY) void k_ref_faces_march(
                 float* const w = second ? w1 : w0;
                 float f[6] = {second ? u1[s] : u0[s], second ? dev::lane_next(u0[s]) : u1[s],
                               v[0], v[S::ROW], w[s], w[s1]};
-                constexpr uint32_t kFull = F_ACTIVE | F_SELF | F_NBRS;
-                relax_full(c == kFull, omega, f);
-                if (c >= F_ACTIVE && c != kFull) relax_partial(c, omega, f);
+                relax_faces(c, diag.of(c), omega, f);
                 v[0] = f[2];
                 v[S::ROW] = f[3];
                 w[s] = f[4];
@@ -323,23 +342,164 @@ __global__ __launch_bounds__(TP * TY) void k_ref_faces_march(
     }
 }
 
-// Half-sweeps per launch and z planes per workgroup of the marched form:
-// one workgroup per CU (1024 threads), whose steps are its planes and the
-// 3H of the pipeline's fill.
-inline int march_planes(const Grid& g, int columns, int h)
+// The pressure form's half-sweeps on a column marched up z: half-sweep h trails
+// half-sweep h-1 by one plane, its cells' z neighbours in this thread's
+// registers, x neighbours in adjacent lanes (DPP), y neighbours in LDS, and
+// one barrier per plane.  The pairs are skewed as above; a cell needs only its
+// neighbours' pressures, so exactly H cells go stale on every side.
+//
+// us per half-sweep, one per launch before: 113x90x101 6.3 -> 3.2, 80^3 4.5 ->
+// 2.6, 256x240x248 44 -> 11.8.  Small grids are a chain of LDS latencies and
+// barriers (16-pair columns, two per CU, then beat 32-pair ones: 48x40x57 2.1
+// against 2.7), large ones 3.5 TB/s of loads and stores over VALU issue.
+template <int TP, int TY, int H>
+struct PressureColumn {
+    static_assert(H % 2 == 0 && 64 % TP == 0, "whole pairs, whole rows per wave");
+    static constexpr int IX = 2 * TP - 2 * H, IY = TY - 2 * H;  // owned cells
+    // Planes in flight: k+1 (entering) down to k-H (below the last relaxed).
+    static constexpr int W = H + 2;
+    static constexpr int ROW = 2 * (TP + 1);     // LDS words of a row: even x, odd x
+    static constexpr int SLOT = (TY + 2) * ROW;  // of a plane, a row more on each side
+};
+
+// `cold`: the pressure starts at zero and is not read.  Cells that are not
+// active are taken, and written, as zero.
+template <int TP, int TY, int H>
+__global__ __launch_bounds__(TP * TY) void k_ref_pressure_march(
+    Grid g, const float* __restrict__ pi, float* __restrict__ po, const float* __restrict__ d,
+    const uint8_t* __restrict__ flags, int zc, int colour, int sweeps, float omega, int cold)
 {
-    int best = g.nz;
-    long long best_cost = -1;
-    for (int chunks = 1; chunks <= (g.nz + 1) / 2; ++chunks) {
-        const int zc = (g.nz + chunks - 1) / chunks;
-        const long long rounds = ((long long)columns * ((g.nz + zc - 1) / zc) + kCUs - 1) / kCUs;
-        const long long cost = rounds * (zc + 3 * h);
-        if (best_cost < 0 || cost < best_cost) {
-            best_cost = cost;
-            best = zc;
+    using S = PressureColumn<TP, TY, H>;
+    constexpr int W = S::W, D = 2;  // D planes of prefetch
+    __shared__ float lp[W * S::SLOT];
+    __shared__ float inv[256];
+    const int t = (int)threadIdx.x, r = (int)threadIdx.y;
+    for (int f = t + TP * r; f < 256; f += TP * TY) inv[f] = dev::cell_inv((uint8_t)f);
+    const int nbx = (int)gridDim.x, nby = (int)gridDim.y;
+    const int b = dev::xcd_tile_order();
+    const int xa = S::IX * (b % nbx) - H, ya = 1 + S::IY * ((b / nbx) % nby) - H;
+    const int z0 = 1 + zc * (b / (nbx * nby)), z1 = min(z0 + zc, g.nz - 1);
+    const int y = ya + r, skew = y & 1, x0 = xa + 2 * t + skew;
+    const bool inside = x0 >= 0 && x0 < g.nx && y >= 0 && y < g.ny;
+    // Lanes outside the grid read its first cells and have no flags.
+    const uint32_t lane = inside ? (uint32_t)g.idx(x0, y, 0) : 0u;
+    const uint32_t fmask = inside ? 0xffffu : 0u;
+    const bool owner = inside && y <= g.ny - 2 && t >= H / 2 && t < TP - H / 2 && r >= H && r < TY - H;
+    // LDS index of the pair's first and second cell in slot 0 (rows from 1).
+    const int l0 = (r + 1) * S::ROW + t + (skew ? TP + 1 : 0);
+    const int l1 = (r + 1) * S::ROW + t + (skew ? 1 : TP + 1);
+
+    float2 p[W], q[W], iv[W];  // pressure, 0 - d * inv, inv (0: not active)
+    float2 np[D], nd[D];
+    uint16_t nf[D];
+    auto load = [&](int z, int s) {
+        const size_t at = (size_t)min(max(z, 0), g.nz - 1) * (size_t)g.plane;
+        if (!cold) __builtin_memcpy(&np[s], pi + at + lane, 8);
+        __builtin_memcpy(&nd[s], d + at + lane, 8);
+        __builtin_memcpy(&nf[s], flags + at + lane, 2);
+    };
+    auto enter = [&](int z, int slot) {  // plane z, prefetched in slot % D
+        const int s = slot % D;
+        const uint32_t c = nf[s] & (z >= 0 && z < g.nz ? fmask : 0u);
+        iv[slot] = make_float2(inv[c & 0xffu], inv[c >> 8]);
+        q[slot] = make_float2(dev::neg_scaled_rhs(nd[s].x, iv[slot].x),
+                              dev::neg_scaled_rhs(nd[s].y, iv[slot].y));
+        p[slot] = make_float2(iv[slot].x > 0.0f ? np[s].x : 0.0f, iv[slot].y > 0.0f ? np[s].y : 0.0f);
+        lp[slot * S::SLOT + l0] = p[slot].x;
+        lp[slot * S::SLOT + l1] = p[slot].y;
+    };
+#pragma unroll
+    for (int s = 0; s < W; ++s) p[s] = q[s] = iv[s] = make_float2(0.0f, 0.0f);
+#pragma unroll
+    for (int s = 0; s < D; ++s) np[s] = make_float2(0.0f, 0.0f);
+    // Step k relaxes plane k - (h-1) for half-sweep h = 1..sweeps.  The first
+    // step's plane is z0 - sweeps (whose plane below is never needed), or one
+    // before for a fixed colour of step 0.
+    int k0 = z0 - sweeps;
+    k0 -= (xa + k0 + colour) & 1;
+    const int kend = z1 + H - 1;  // one past the step that writes plane z1 - 1
+#pragma unroll
+    for (int s = 0; s < D; ++s) load(k0 + s, s);
+    __syncthreads();  // inv
+    enter(k0, 0);
+    load(k0 + D, 0);
+    __syncthreads();
+    for (int kb = k0; kb < kend; kb += W) {
+#pragma unroll
+        for (int u = 0; u < W; ++u) {
+            const int k = kb + u;  // in slot u
+            if (k >= kend) break;
+            enter(k + 1, (u + 1) % W);
+            load(k + 1 + D, (u + 1) % W % D);
+            const bool second = u & 1;  // the pair's cell of this step's colour
+            // The y neighbours of every half-sweep's cell, none of which this
+            // step changes, in one go.
+            float yn[H][2];
+#pragma unroll
+            for (int h = 1; h <= H; ++h) {
+                const float* const at = lp + (u - (h - 1) + W) % W * S::SLOT + (second ? l1 : l0);
+                yn[h - 1][0] = at[-S::ROW];
+                yn[h - 1][1] = at[S::ROW];
+            }
+#pragma unroll
+            for (int h = 1; h <= H; ++h) {
+                const int z = k - (h - 1);
+                // Planes whose cells half-sweep h must relax.
+                if (h > sweeps || z < z0 - (sweeps - h) || z > z1 - 1 + (sweeps - h)) continue;
+                const int s = (u - (h - 1) + W) % W, lo = (s + W - 1) % W, hi = (s + 1) % W;
+                const float left = second ? p[s].x : dev::lane_prev(p[s].y);
+                const float right = second ? dev::lane_next(p[s].x) : p[s].y;
+                const float pc = second ? p[s].y : p[s].x;
+                const float w = second ? iv[s].y : iv[s].x;
+                const float sum = dev::sum6(left, right, yn[h - 1][0], yn[h - 1][1],
+                                            second ? p[lo].y : p[lo].x, second ? p[hi].y : p[hi].x);
+                const float G = __builtin_fmaf(sum, w, second ? q[s].y : q[s].x);
+                const float v = pc + omega * (G - pc);
+                const float out = w > 0.0f ? v : pc;
+                if (second) p[s].y = out;
+                else p[s].x = out;
+                lp[s * S::SLOT + (second ? l1 : l0)] = out;
+            }
+            const int zo = k - (H - 1);
+            if (zo >= z0 && owner)
+                __builtin_memcpy(po + (size_t)zo * (size_t)g.plane + lane, &p[(u - (H - 1) + W) % W], 8);
+            __syncthreads();
         }
     }
-    return best;
+}
+
+// Planes per workgroup of the marched forms, one workgroup per CU (1024
+// threads), and the steps of the busiest CU: a workgroup's steps are its planes
+// and the pipeline's fill.
+struct MarchPlan {
+    dim3 grid;
+    int zc;
+    long long steps;
+};
+inline MarchPlan march_plan(int nx, int ny, int planes, int fill)
+{
+    MarchPlan p = {dim3(), planes, -1};
+    for (int chunks = 1; chunks <= (planes + 1) / 2; ++chunks) {
+        const int zc = (planes + chunks - 1) / chunks;
+        const long long rounds = ((long long)nx * ny * ((planes + zc - 1) / zc) + kCUs - 1) / kCUs;
+        const long long steps = rounds * (zc + fill);
+        if (p.steps < 0 || steps < p.steps) {
+            p.steps = steps;
+            p.zc = zc;
+        }
+    }
+    p.grid = dim3((unsigned)nx, (unsigned)ny, (unsigned)((planes + p.zc - 1) / p.zc));
+    return p;
+}
+
+constexpr int kMarchTP = 32, kMarchTY = 32;
+
+template <int H>
+MarchPlan faces_plan(const Grid& g)
+{
+    using S = FaceColumn<kMarchTP, kMarchTY, H>;
+    // Odd rows may own one x less on the right: columns for nx + 1.
+    return march_plan((g.nx + S::IX) / S::IX, (g.ny + S::IY - 1) / S::IY, g.nz, 3 * H);
 }
 
 struct FaceSets {
@@ -351,14 +511,29 @@ template <int H>
 hipError_t launch_faces_march(const Grid& g, const FaceSets& f, const uint8_t* flags, int colour,
                               int sweeps, double omega, hipStream_t st)
 {
-    constexpr int TP = 32, TY = 32;
-    using S = FaceColumn<TP, TY, H>;
-    // Odd rows own one x less on the right: columns for nx + 1.
-    const int nx = (g.nx + S::IX) / S::IX, ny = (g.ny + S::IY - 1) / S::IY;
-    const int zc = march_planes(g, nx * ny, H);
-    const dim3 grid((unsigned)nx, (unsigned)ny, (unsigned)((g.nz + zc - 1) / zc));
-    hipLaunchKernelGGL((k_ref_faces_march<TP, TY, H>), grid, dim3(TP, TY), 0, st, g, f.ui, f.vi,
-                       f.wi, f.uo, f.vo, f.wo, flags, zc, colour, sweeps, omega);
+    const MarchPlan p = faces_plan<H>(g);
+    const int zc = p.zc;
+    hipLaunchKernelGGL((k_ref_faces_march<kMarchTP, kMarchTY, H>), p.grid, dim3(kMarchTP, kMarchTY), 0,
+                       st, g, f.ui, f.vi, f.wi, f.uo, f.vo, f.wo, flags, zc, colour, sweeps, omega);
+    return hipGetLastError();
+}
+
+template <int TP, int H>
+MarchPlan pressure_plan(const Grid& g)
+{
+    using S = PressureColumn<TP, kMarchTY, H>;
+    return march_plan((g.nx - 1 + S::IX - 1) / S::IX, (g.ny - 2 + S::IY - 1) / S::IY, g.nz - 2, 2 * H);
+}
+
+template <int TP, int H>
+hipError_t launch_pressure_march(const Grid& g, const float* pi, float* po, const float* d,
+                                 const uint8_t* flags, int colour, int sweeps, float omega, int cold,
+                                 hipStream_t st)
+{
+    const MarchPlan p = pressure_plan<TP, H>(g);
+    const int zc = p.zc;
+    hipLaunchKernelGGL((k_ref_pressure_march<TP, kMarchTY, H>), p.grid, dim3(TP, kMarchTY), 0, st, g, pi,
+                       po, d, flags, zc, colour, sweeps, omega, cold);
     return hipGetLastError();
 }
 

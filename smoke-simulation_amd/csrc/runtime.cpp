@@ -499,18 +499,20 @@ hipError_t stage_project(smoke_sim* s, long long* launches)
         *launches += sweep_launches;
         if ((e = sweep_mark(s, 1, sweep_launches)) != hipSuccess) return e;
     } else {
-        if (p.warm_start) e = smk::mask_pressure(g, s->P[s->pcur], s->flags, s->stream);
-        else e = smk::fill_f32(s->P[s->pcur], g.elems, 0.0f, s->stream);
-        if (e != hipSuccess) return e;
-        *launches += 1;
+        int n_launches = 0;
+        if (p.iterations == 0) {
+            // No half-sweeps: P = 0, or the last step's on the active cells.
+            e = p.warm_start ? smk::mask_pressure(g, s->P[s->pcur], s->flags, s->stream)
+                             : smk::fill_f32(s->P[s->pcur], g.elems, 0.0f, s->stream);
+            if (e != hipSuccess) return e;
+            *launches += 1;
+        }
         if ((e = sweep_mark(s, 0, 0)) != hipSuccess) return e;
-        for (int it = 0; it < p.iterations; ++it)
-            for (int o = 0; o < 2; ++o) {
-                e = smk::rbsor_half(g, s->P[s->pcur], s->d, s->flags, o, (float)p.sor_omega, s->stream);
-                if (e != hipSuccess) return e;
-                *launches += 1;
-            }
-        if ((e = sweep_mark(s, 1, 2LL * p.iterations)) != hipSuccess) return e;
+        e = smk::rbsor_sweeps(g, s->P, &s->pcur, s->d, s->flags, 2 * p.iterations, (float)p.sor_omega,
+                              !p.warm_start, s->stream, &n_launches);
+        if (e != hipSuccess) return e;
+        *launches += n_launches;
+        if ((e = sweep_mark(s, 1, n_launches)) != hipSuccess) return e;
     }
     e = smk::with_fields(s, [&](auto, auto u, auto v, auto w) {
         return smk::gradient(g, u[n], v[n], w[n], s->P[s->pcur], s->flags, s->stream);

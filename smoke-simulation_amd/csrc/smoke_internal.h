@@ -301,8 +301,12 @@ hipError_t jacobi_sweep(const Grid& g, const float* pin, float* pout, const floa
 hipError_t jacobi_fused(const Grid& g, const float* pin, float* pout, const float* d,
                         const uint8_t* flags, const JacobiPlan& plan, int sweeps, float omega,
                         int plain, int zero_in, hipStream_t st);
-hipError_t rbsor_half(const Grid& g, float* p, const float* d, const uint8_t* flags, int colour,
-                      float omega, hipStream_t st);
+// `sweeps` half-sweeps of the pressure form, several per launch (redblack.h),
+// from p[*cur] (cold: from zero; cells that are not active count as zero),
+// ping-ponging the two buffers; the result is in p[*cur].
+hipError_t rbsor_sweeps(const Grid& g, float* const (&p)[2], int* cur, const float* d,
+                        const uint8_t* flags, int sweeps, float omega, int cold, hipStream_t st,
+                        int* launches);
 hipError_t mask_pressure(const Grid& g, float* p, const uint8_t* flags, hipStream_t st);
 hipError_t gradient(const Grid& g, float* u, float* v, float* w, const float* p,
                     const uint8_t* flags, hipStream_t st);

@@ -360,54 +360,6 @@ __global__ __launch_bounds__(TX * TY / R, 8 / R) void k_jacobi_fused(
                                                  L % nbx, (L / nbx) % nby, L / (nbx * nby), sh);
 }
 
-// One red-black SOR half-sweep of the pressure form, in place.
-__global__ __launch_bounds__(BX * BY) void k_rbsor_half(Grid g, float* __restrict__ p,
-                                                    const float* __restrict__ d,
-                                                    const uint8_t* __restrict__ flags, int colour,
-                                                    float omega, int pairs)
-{
-    // The same thread layout as k_project_ref_half: a flat (column pair, row)
-    // index and kRefZ consecutive planes per thread, every load issued before
-    // any update.  The neighbours are of the other colour, which this launch
-    // leaves alone, and every interior cell's neighbours lie inside the array.
-    const int f = (int)blockIdx.x * (BX * BY) + (int)threadIdx.y * BX + (int)threadIdx.x;
-    if (f >= pairs * (g.ny - 2)) return;
-    const int t = f % pairs, y = f / pairs + 1;
-    const int z0 = (int)blockIdx.y * kRefZ + 1;
-    float nb[kRefZ][6], pc[kRefZ], di[kRefZ];
-    uint8_t fl[kRefZ];
-    int ic[kRefZ];
-#pragma unroll
-    for (int j = 0; j < kRefZ; ++j) {
-        const int z = z0 + j, x = dev::colour_x(t, y, z, colour);
-        fl[j] = 0;
-        ic[j] = 0;
-        pc[j] = di[j] = 0.0f;
-#pragma unroll
-        for (int k = 0; k < 6; ++k) nb[j][k] = 0.0f;
-        if (z > g.nz - 2 || x > g.nx - 2) continue;
-        const int i = g.idx(x, y, z);
-        ic[j] = i;
-        nb[j][0] = p[i - 1];
-        nb[j][1] = p[i + 1];
-        nb[j][2] = p[i - g.px];
-        nb[j][3] = p[i + g.px];
-        nb[j][4] = p[i - g.plane];
-        nb[j][5] = p[i + g.plane];
-        pc[j] = p[i];
-        di[j] = d[i];
-        fl[j] = flags[i];
-    }
-#pragma unroll
-    for (int j = 0; j < kRefZ; ++j) {
-        if (!(fl[j] & F_ACTIVE)) continue;
-        const float G = dev::pressure_update(
-            dev::sum6(nb[j][0], nb[j][1], nb[j][2], nb[j][3], nb[j][4], nb[j][5]),
-            dev::inv_acc(__popc(fl[j] & F_NBRS)), di[j]);
-        p[ic[j]] = pc[j] + omega * (G - pc[j]);
-    }
-}
-
 // Warm start: zero the pressure of cells that are not active.
 __global__ void k_mask_pressure(Grid g, float* __restrict__ p, const uint8_t* __restrict__ flags)
 {
@@ -673,18 +625,21 @@ hipError_t project_reference_sweeps(const Grid& g, float* const (&a)[3], float* 
                                     const uint8_t* flags, int sweeps, double omega, hipStream_t st,
                                     int* launches)
 {
-    // At most one box per CU: boxes (redblack.h has both sides).  Else columns:
-    // 6 half-sweeps per launch where the two sets of faces and the flags
+    // At most one box per CU: boxes (redblack.h has both sides).  Else columns,
+    // 4 half-sweeps per launch, or where the two sets of faces and the flags
     // approach the 256 MB memory-side cache (a launch is then bound by memory
-    // and fewer passes pay for the larger halo), 4 where they do not.  us per
-    // half-sweep with 4 / 6: 160^3 (125 MB) 8.1 / 8.4, 192x180x188 (191 MB)
-    // 10.7 / 10.2, 224x200x210 (271 MB) 18.0 / 14.1, 256x240x248 29.8 / 22.4.
+    // and fewer passes pay for the larger halo) the better fitting of 5 and 6.
+    // us per half-sweep with 4 / 5 / 6: 160^3 (125 MB) 8.6 / 10.0 / 9.5,
+    // 192x180x188 (191 MB) 11.6 / 11.9 / 11.7, 224x200x210 (271 MB) 19.7 /
+    // 16.9 / 16.0, 256x240x248 29.4 / 26.6 / 29.0 (one column more for 6).
     constexpr int IX = 24, IY = 10, IZ = 10;
     const dim3 boxes((unsigned)((g.nx + IX - 1) / IX), (unsigned)((g.ny + IY - 1) / IY),
                      (unsigned)((g.nz + IZ - 1) / IZ));
     const bool boxed = (long long)boxes.x * boxes.y * boxes.z <= kCUs;
-    const bool large = (long long)g.elems * 25 > (150LL << 20);
-    const int H = !boxed && large ? 6 : 4;
+    const bool large = (long long)g.elems * 25 > (180LL << 20);
+    int H = 4;
+    if (!boxed && large)
+        H = faces_plan<5>(g).steps * 6 < faces_plan<6>(g).steps * 5 ? 5 : 6;
     // An even number of launches, so that the last one writes a again.
     const int n = 2 * ((sweeps + 2 * H - 1) / (2 * H));
     *launches = 0;
@@ -699,8 +654,9 @@ hipError_t project_reference_sweeps(const Grid& g, float* const (&a)[3], float* 
                                f.ui, f.vi, f.wi, f.uo, f.vo, f.wo, flags, colour, m, omega);
             e = hipGetLastError();
         } else {
-            e = large ? launch_faces_march<6>(g, f, flags, colour, m, omega, st)
-                      : launch_faces_march<4>(g, f, flags, colour, m, omega, st);
+            e = H == 6   ? launch_faces_march<6>(g, f, flags, colour, m, omega, st)
+                : H == 5 ? launch_faces_march<5>(g, f, flags, colour, m, omega, st)
+                         : launch_faces_march<4>(g, f, flags, colour, m, omega, st);
         }
         if (e != hipSuccess) return e;
         done += m;
@@ -829,16 +785,34 @@ hipError_t jacobi_fused(const Grid& g, const float* pin, float* pout, const floa
     }
 }
 
-hipError_t rbsor_half(const Grid& g, float* p, const float* d, const uint8_t* flags, int colour,
-                      float omega, hipStream_t st)
+hipError_t rbsor_sweeps(const Grid& g, float* const (&p)[2], int* cur, const float* d,
+                        const uint8_t* flags, int sweeps, float omega, int cold, hipStream_t st,
+                        int* launches)
 {
-    const int pairs = (g.nx - 2 + 1) / 2;
-    const long long items = (long long)pairs * (g.ny - 2);
-    const dim3 grid((unsigned)((items + BX * BY - 1) / (BX * BY)),
-                    (unsigned)((g.nz - 2 + kRefZ - 1) / kRefZ));
-    hipLaunchKernelGGL(k_rbsor_half, grid, dim3(BX, BY), 0, st, g, p, d, flags, colour, omega,
-                       pairs);
-    return hipGetLastError();
+    // 4 or 6 half-sweeps per launch, whichever takes fewer steps per
+    // half-sweep; narrow columns where the grid is too small to fill the CUs
+    // with wide ones.  us per half-sweep, narrow 4 / 4 / 6: 48x40x57 2.1 / 2.8
+    // / 2.7, 80^3 2.6 / 2.9 / 2.8, 113x90x101 3.2 / 3.3 / 3.4, 150^3 4.8 / 5.0 /
+    // 4.7, 256x240x248 13.3 / 12.3 / 11.8.
+    const bool narrow = (long long)g.nx * g.ny * g.nz <= 1500000;
+    const int H = narrow || pressure_plan<32, 4>(g).steps * 6 <= pressure_plan<32, 6>(g).steps * 4 ? 4 : 6;
+    const int n = (sweeps + H - 1) / H;
+    *launches = 0;
+    for (int l = 0, done = 0; l < n; ++l) {
+        const int m = sweeps / n + (l < sweeps % n ? 1 : 0), colour = done & 1;
+        const float* pi = p[*cur];
+        float* po = p[*cur ^ 1];
+        const int zero_in = cold && l == 0;
+        const hipError_t e =
+            narrow   ? launch_pressure_march<16, 4>(g, pi, po, d, flags, colour, m, omega, zero_in, st)
+            : H == 4 ? launch_pressure_march<32, 4>(g, pi, po, d, flags, colour, m, omega, zero_in, st)
+                     : launch_pressure_march<32, 6>(g, pi, po, d, flags, colour, m, omega, zero_in, st);
+        if (e != hipSuccess) return e;
+        *cur ^= 1;
+        done += m;
+        ++*launches;
+    }
+    return hipSuccess;
 }
 
 hipError_t mask_pressure(const Grid& g, float* p, const uint8_t* flags, hipStream_t st)

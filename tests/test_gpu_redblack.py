@@ -11,9 +11,9 @@ from smokesim import scenes
 pytestmark = pytest.mark.gpu
 
 # One box, full and cut boxes, then columns (more than 256 boxes) whole and cut
-# in x, y and z, and the largest with more half-sweeps per launch.
+# in x, y and z, and the largest with 6 half-sweeps per launch (5: test_gpu_full_size).
 DIMS = [(3, 3, 3), (4, 11, 10), (24, 10, 10), (25, 11, 21), (47, 20, 9), (49, 31, 33), (97, 40, 12),
-        (56, 96, 120), (113, 75, 74), (3, 640, 90), (241, 161, 150)]
+        (56, 96, 120), (113, 75, 74), (3, 640, 90), (241, 200, 150)]
 
 
 def scene(dims, projection, iterations, **params):
@@ -33,6 +33,24 @@ def test_reference_form(dims, iterations):
         g.step(sc["dt"], readback=False)
         o.step(sc["dt"])
         assert_bitwise_equal(g.state(), o.state(), f"{dims} x{iterations} step {k}")
+    g.close()
+
+
+@pytest.mark.parametrize("dims", DIMS, ids=str)
+@pytest.mark.parametrize("iterations,warm", [(1, 0), (2, 1), (3, 1), (13, 0)])
+def test_pressure_form(dims, iterations, warm):
+    sc = scene(dims, smokesim.PROJ_RBSOR, iterations, warm_start=warm)
+    dens = random_density(dims, 4)
+    g, o = gpu_for(sc, dens), oracle_for(sc, 32, dens)
+    for k in range(3):
+        if k == 2:  # cells that become solid lose their pressure
+            for s in (g, o):
+                s.move_object(0, dims[0] / 2, dims[1] / 2, dims[2] / 2)
+        g.step(sc["dt"], readback=False)
+        o.step(sc["dt"])
+        assert_bitwise_equal(g.state(), o.state(), f"{dims} x{iterations} step {k}")
+        assert np.array_equal(g.get_pressure().view(np.uint32),
+                              o.get_pressure().astype(np.float32).view(np.uint32))
     g.close()
 
 
