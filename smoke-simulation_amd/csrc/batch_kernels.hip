@@ -116,9 +116,10 @@ __global__ __launch_bounds__(BX * BY) void kb_adv_v(const SimDesc* __restrict__ 
         const int gx = tab->gx[si], gy = tab->gy[si];
         const SimDesc& s = sims[si];
         const int n = s.now, p = 1 - s.now;
-        dev::advect_velocity_march<BY, kAdvChunkZ>(
+        dev::advect_velocity_march<BY>(
             s.g, s.u[n], s.v[n], s.w[n], s.u[p], s.v[p], s.w[p], s.flags, s.force.dt,
-            1 + BX * (lb % gx), 1 + BY * ((lb / gx) % gy), 1 + kAdvChunkZ * (lb / (gx * gy)), ring);
+            1 + BX * (lb % gx), 1 + BY * ((lb / gx) % gy), 1 + kAdvChunkZ * (lb / (gx * gy)),
+            kAdvChunkZ, ring);
         __syncthreads();
     }
 }
@@ -137,9 +138,10 @@ __global__ __launch_bounds__(BX * BY) void kb_adv_d(const SimDesc* __restrict__ 
         const int gx = tab->gx[si], gy = tab->gy[si];
         const SimDesc& s = sims[si];
         const int n = s.now, p = 1 - s.now;
-        dev::advect_density_march<BY, kAdvChunkZ>(
+        dev::advect_density_march<BY>(
             s.g, s.rho[n], s.rho[p], s.u[p], s.v[p], s.w[p], s.flags, s.force.dt, BX * (lb % gx),
-            1 + BY * ((lb / gx) % gy), 1 + kAdvChunkZ * (lb / (gx * gy)), ring);
+            1 + BY * ((lb / gx) % gy), 1 + kAdvChunkZ * (lb / (gx * gy)),
+            kAdvChunkZ, ring);
         __syncthreads();
     }
 }

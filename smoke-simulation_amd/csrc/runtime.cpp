@@ -317,18 +317,14 @@ using smk::refresh_mask;
 hipError_t stage_scene(smoke_sim* s, long long* launches)
 {
     s->now = 1 - s->now;  // smokeSimulation.cu:777-779
-    for (const Object& o : s->objects) {
-        if (o.type != 1) continue;
-        int launched = 0;
-        hipError_t e = smk::with_fields(s, [&](auto rho, auto, auto, auto) {
-            return smk::fill_source(s->g, rho[0], rho[1],
-                                    make_float4(o.pos[0], o.pos[1], o.pos[2], o.r), s->stream,
-                                    &launched);
-        });
-        if (e != hipSuccess) return e;
-        *launches += launched;
-    }
-    hipError_t e = refresh_mask(s, launches);
+    const smk::SphereList src = sphere_list(s, 1);
+    int launched = 0;
+    hipError_t e = smk::with_fields(s, [&](auto rho, auto, auto, auto) {
+        return smk::fill_sources(s->g, rho[0], rho[1], src, s->stream, &launched);
+    });
+    if (e != hipSuccess) return e;
+    *launches += launched;
+    e = refresh_mask(s, launches);
     if (e != hipSuccess || !s->prm.obstacle_velocity) return e;
     if (!s->owner) return hipErrorNotInitialized;  // set_params allocates it
     smk::SphereList vel;

@@ -239,8 +239,9 @@ hipError_t floor_mask(const Grid& g, uint8_t* base, hipStream_t st);
 hipError_t build_mask(const Grid& g, const uint8_t* base, uint8_t* s, const SphereList& obst,
                       int mode, hipStream_t st);
 hipError_t build_flags(const Grid& g, const uint8_t* s, uint8_t* flags, hipStream_t st);
-hipError_t fill_source(const Grid& g, float* rho0, float* rho1, float4 sph, hipStream_t st,
-                       int* launched);
+// Every source's cells to 1 in both halves; *launched: the launches it took.
+hipError_t fill_sources(const Grid& g, float* rho0, float* rho1, const SphereList& src, hipStream_t st,
+                        int* launched);
 // Conservative bounding box of a source sphere clipped to the interior:
 // false if it holds no cell.
 bool source_box(const Grid& g, float4 sph, int lo[3], int ext[3]);
@@ -329,8 +330,8 @@ hipError_t advect_density(const Grid& g, const float* r0, float* r1, const float
     hipError_t pack_faces_f32(const Grid& g, const H* src, float* dst, hipStream_t st);            \
     hipError_t pack_cells_half(const Grid& g, const H* src, uint16_t* dst, int format,             \
                                hipStream_t st);                                                    \
-    hipError_t fill_source(const Grid& g, H* rho0, H* rho1, float4 sph, hipStream_t st,            \
-                           int* launched);                                                         \
+    hipError_t fill_sources(const Grid& g, H* rho0, H* rho1, const SphereList& src,                \
+                            hipStream_t st, int* launched);                                        \
     hipError_t force(const Grid& g, H* u, H* v, H* w, const H* rho, const uint8_t* flags,          \
                      const ForceArgs& a, hipStream_t st);                                          \
     hipError_t force(const Grid& g, H* u, H* v, H* w, const float* rho, const uint8_t* flags,      \

@@ -920,7 +920,7 @@ __device__ __forceinline__ float tri_ring(const T* __restrict__ a, const float* 
 }
 
 // advect_velocity_at over a column of BX x AY cells at (x0, y0), z in
-// [z0, min(z0 + ZC, nz) - 1], with a block of BX x AY threads (AY == BY):
+// [z0, min(z0 + zc, nz) - 1], with a block of BX x AY threads (AY == BY):
 // the block marches up z keeping window planes z-1, z, z+1 of u, v, w in a
 // 4-slot LDS ring; while plane z is computed, window plane z+2 is loaded into
 // registers and then stored into the slot of plane z-2 (last read in the
@@ -930,14 +930,14 @@ __device__ __forceinline__ float tri_ring(const T* __restrict__ a, const float* 
 // thread has one cell per plane.  Window rows/columns past (ny, nx) are left
 // at zero and never read; window planes stay at or below nz.  Same values,
 // same arithmetic as advect_velocity_at: the results are identical.
-template <int AY, int ZC, typename T>
+template <int AY, typename T>
 __device__ __forceinline__ void advect_velocity_march(const Grid& g, const T* __restrict__ u0,
                                                       const T* __restrict__ v0,
                                                       const T* __restrict__ w0,
                                                       T* __restrict__ u1, T* __restrict__ v1,
                                                       T* __restrict__ w1,
                                                       const uint8_t* __restrict__ flags, float dt,
-                                                      int x0, int y0, int z0,
+                                                      int x0, int y0, int z0, int zc,
                                                       AdvRing<BX, AY, 4, 3>& ring)
 {
     static_assert(AY == BY, "one cell per thread and plane");
@@ -947,7 +947,7 @@ __device__ __forceinline__ void advect_velocity_march(const Grid& g, const T* __
     const T* const src[3] = {u0, v0, w0};
     const int wx0 = x0 - 1, wy0 = y0 - 1;
     const int x = x0 + (int)threadIdx.x, y = y0 + (int)threadIdx.y;
-    const int zlast = min(z0 + ZC, g.nz) - 1;  // the grid keeps z0 <= nz - 1
+    const int zlast = min(z0 + zc, g.nz) - 1;  // the grid keeps z0 <= nz - 1
     const bool col = x <= g.nx - 1 && y <= g.ny - 1;
     {
         const P a = ring_load<BX, AY, NR, 3, 1>(g, src, wx0, wy0, z0 - 1);
@@ -1046,7 +1046,7 @@ __device__ __forceinline__ void advect_density_col(const Grid& g, const T* __res
         if (self[j]) stf(r1, g.idx(x, y, z0 + j), s[j]);
 }
 // advect_density_col over a column of BX x AY cells at (x0, y0), z in
-// [z0, min(z0 + ZC, nz - 1) - 1], with a block of BX x AY threads
+// [z0, min(z0 + zc, nz - 1) - 1], with a block of BX x AY threads
 // (AY == BY; x0 a multiple of BX, lane x = cell x, lane 0 of the first
 // column idle), marching up z like advect_velocity_march: window planes z-1,
 // z, z+1 of the density (x in [x0-2, x0+BX+1], y in [y0-1, y0+AY]: the column
@@ -1054,13 +1054,13 @@ __device__ __forceinline__ void advect_density_col(const Grid& g, const T* __res
 // plane z is computed.  Samples whose corners lie in the ring read LDS, a
 // back-trace longer than one cell reads global memory.  Same values, same
 // arithmetic as advect_density_col: the results are identical.
-template <int AY, int ZC, typename T, typename TV>
+template <int AY, typename T, typename TV>
 __device__ __forceinline__ void advect_density_march(const Grid& g, const T* __restrict__ r0,
                                                      T* __restrict__ r1, const TV* __restrict__ u,
                                                      const TV* __restrict__ v,
                                                      const TV* __restrict__ w,
                                                      const uint8_t* __restrict__ flags, float dt,
-                                                     int x0, int y0, int z0,
+                                                     int x0, int y0, int z0, int zc,
                                                      AdvRing<BX, AY, 4, 1, 2>& ring)
 {
     static_assert(AY == BY, "one cell per thread and plane");
@@ -1070,7 +1070,7 @@ __device__ __forceinline__ void advect_density_march(const Grid& g, const T* __r
     const T* const src[1] = {r0};
     const int wx0 = x0 - 2, wy0 = y0 - 1;
     const int x = x0 + (int)threadIdx.x, y = y0 + (int)threadIdx.y;
-    const int zlast = min(z0 + ZC, g.nz - 1) - 1;  // the grid keeps z0 <= nz - 2
+    const int zlast = min(z0 + zc, g.nz - 1) - 1;  // the grid keeps z0 <= nz - 2
     const bool col = x >= 1 && x <= g.nx - 2 && y <= g.ny - 2;
     // Faces and flags of cell z (loaded one plane ahead).
     struct Faces {

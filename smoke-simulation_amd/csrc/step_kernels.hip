@@ -221,17 +221,24 @@ __global__ void k_obstacle_bc(Grid g, T* __restrict__ u, T* __restrict__ v, T* _
     }
 }
 
-// fillSmoke (smokeSimulation.cu:251-273) restricted to the bounding box of
-// one source (clipped to the interior by the launcher).
+// fillSmoke (smokeSimulation.cu:251-273) for every source in one launch,
+// restricted to the sources' bounding boxes (clipped to the interior by the
+// launcher): blockIdx.z counts their planes, source after source.
+struct SourceBoxes {
+    int count;
+    int first[SMOKE_MAX_OBJECTS + 1];  // planes of the sources before
+    int lo[SMOKE_MAX_OBJECTS][3], ext[SMOKE_MAX_OBJECTS][2];
+    float4 s[SMOKE_MAX_OBJECTS];
+};
 template <typename T>
-__global__ void k_source(Grid g, T* __restrict__ r0, T* __restrict__ r1, float4 sph, int x0, int y0,
-                         int z0, int ex, int ey)
+__global__ void k_source(Grid g, T* __restrict__ r0, T* __restrict__ r1, SourceBoxes b)
 {
-    int x = x0 + blockIdx.x * BX + threadIdx.x;
-    int y = y0 + blockIdx.y * BY + threadIdx.y;
-    int z = z0 + blockIdx.z;
-    if (x >= x0 + ex || y >= y0 + ey) return;
-    dev::source_at(g, r0, r1, sph, x, y, z);
+    int k = 0;
+    while (b.first[k + 1] <= (int)blockIdx.z) ++k;
+    const int lx = blockIdx.x * BX + threadIdx.x, ly = blockIdx.y * BY + threadIdx.y;
+    if (lx >= b.ext[k][0] || ly >= b.ext[k][1]) return;
+    dev::source_at(g, r0, r1, b.s[k], b.lo[k][0] + lx, b.lo[k][1] + ly,
+                   b.lo[k][2] + (int)blockIdx.z - b.first[k]);
 }
 
 // ---------------------------------------------------------- step stages
@@ -380,36 +387,47 @@ __global__ void k_gradient(Grid g, T* __restrict__ u, T* __restrict__ v, T* __re
 }
 
 // Velocity advection: a block of BX x BY threads marches a column of BX x BY
-// cells through kAdvZC planes (dev::advect_velocity_march), in XCD tile order.
-constexpr int kAdvZC = kAdvChunkZ;
-
+// cells through zc planes (dev::advect_velocity_march), in XCD tile order.
 template <typename T>
 __global__ __launch_bounds__(BX * BY) void k_advect_velocity(
     Grid g, const T* __restrict__ u0, const T* __restrict__ v0, const T* __restrict__ w0,
     T* __restrict__ u1, T* __restrict__ v1, T* __restrict__ w1, const uint8_t* __restrict__ flags,
-    float dt)
+    float dt, int zc)
 {
     __shared__ dev::AdvRing<BX, BY, 4, 3> ring;
     const int nbx = (int)gridDim.x, nby = (int)gridDim.y;
     const int L = dev::xcd_tile_order();
-    dev::advect_velocity_march<BY, kAdvZC>(g, u0, v0, w0, u1, v1, w1, flags, dt,
-                                           1 + BX * (L % nbx), 1 + BY * ((L / nbx) % nby),
-                                           1 + kAdvZC * (L / (nbx * nby)), ring);
+    dev::advect_velocity_march<BY>(g, u0, v0, w0, u1, v1, w1, flags, dt, 1 + BX * (L % nbx),
+                                   1 + BY * ((L / nbx) % nby), 1 + zc * (L / (nbx * nby)), zc, ring);
 }
 
 // Density advection: a block of BX x BY threads marches a column of BX x BY
-// cells through kAdvZC planes (dev::advect_density_march), in XCD tile order.
+// cells through zc planes (dev::advect_density_march), in XCD tile order.
 template <typename T, typename TV>
 __global__ __launch_bounds__(BX * BY) void k_advect_density(
     Grid g, const T* __restrict__ r0, T* __restrict__ r1, const TV* __restrict__ u,
-    const TV* __restrict__ v, const TV* __restrict__ w, const uint8_t* __restrict__ flags, float dt)
+    const TV* __restrict__ v, const TV* __restrict__ w, const uint8_t* __restrict__ flags, float dt,
+    int zc)
 {
     __shared__ dev::AdvRing<BX, BY, 4, 1, 2> ring;
     const int nbx = (int)gridDim.x, nby = (int)gridDim.y;
     const int L = dev::xcd_tile_order();
-    dev::advect_density_march<BY, kAdvZC>(g, r0, r1, u, v, w, flags, dt, BX * (L % nbx),
-                                          1 + BY * ((L / nbx) % nby),
-                                          1 + kAdvZC * (L / (nbx * nby)), ring);
+    dev::advect_density_march<BY>(g, r0, r1, u, v, w, flags, dt, BX * (L % nbx),
+                                  1 + BY * ((L / nbx) % nby), 1 + zc * (L / (nbx * nby)), zc, ring);
+}
+
+// Planes per block of the marched advection: kAdvChunkZ, fewer (down to 2)
+// while the blocks would not give every CU four.  A block's planes are a serial
+// chain of about 1.4 us each, so a grid that does not fill the GPU takes less
+// time in shorter chunks although their window planes are loaded more often.
+// Velocity / density, chunks of 16 -> this rule, us: 48x40x57 23.0 -> 6.0 / 15.7
+// -> 4.1, 80^3 26.1 -> 11.0 / 16.9 -> 7.2, 113x90x101 28.8 -> 15.3 / 18.5 -> 9.1,
+// 150x96x121 33.1 -> 25.1 / 20.4 -> 14.7 (two per CU: 13.8 / 7.6 at 80^3).
+inline int advect_chunk(const dim3& columns, int planes)
+{
+    int zc = kAdvChunkZ;
+    while (zc > 2 && (long long)columns.x * columns.y * ((planes + zc - 1) / zc) < 4 * kCUs) zc /= 2;
+    return zc;
 }
 
 }  // namespace
@@ -553,22 +571,45 @@ bool source_box(const Grid& g, float4 sph, int lo[3], int ext[3])
 }
 
 template <typename T>
-static hipError_t launch_source(const Grid& g, T* rho0, T* rho1, float4 sph, hipStream_t st,
-                               int* launched)
+static hipError_t launch_sources(const Grid& g, T* rho0, T* rho1, const SphereList& src,
+                                 hipStream_t st, int* launched)
 {
     *launched = 0;
-    int lo[3], ext[3];
-    if (!source_box(g, sph, lo, ext)) return hipSuccess;
-    hipLaunchKernelGGL(k_source<T>, grid_for(ext[0], ext[1], ext[2]), dim3(BX, BY), 0, st, g, rho0,
-                       rho1, sph, lo[0], lo[1], lo[2], ext[0], ext[1]);
-    *launched = 1;
-    return hipGetLastError();
+    SourceBoxes b;
+    b.count = 0;
+    b.first[0] = 0;
+    int wx = 0, wy = 0;
+    auto launch = [&]() {
+        if (b.count == 0) return hipSuccess;
+        hipLaunchKernelGGL(k_source<T>, grid_for(wx, wy, b.first[b.count]), dim3(BX, BY), 0, st, g, rho0,
+                           rho1, b);
+        *launched += 1;
+        b.count = wx = wy = 0;
+        return hipGetLastError();
+    };
+    for (int k = 0; k < src.count; ++k) {
+        int lo[3], ext[3];
+        if (!source_box(g, src.s[k], lo, ext)) continue;
+        if (b.first[b.count] + (long long)ext[2] > 65535) {  // a grid's z extent
+            const hipError_t e = launch();
+            if (e != hipSuccess) return e;
+        }
+        const int n = b.count++;
+        for (int a = 0; a < 3; ++a) b.lo[n][a] = lo[a];
+        b.ext[n][0] = ext[0];
+        b.ext[n][1] = ext[1];
+        b.s[n] = src.s[k];
+        b.first[n + 1] = b.first[n] + ext[2];
+        wx = std::max(wx, ext[0]);
+        wy = std::max(wy, ext[1]);
+    }
+    return launch();
 }
 
-hipError_t fill_source(const Grid& g, float* rho0, float* rho1, float4 sph, hipStream_t st,
-                       int* launched)
+hipError_t fill_sources(const Grid& g, float* rho0, float* rho1, const SphereList& src, hipStream_t st,
+                        int* launched)
 {
-    return launch_source(g, rho0, rho1, sph, st, launched);
+    return launch_sources(g, rho0, rho1, src, st, launched);
 }
 
 template <typename T, typename TR>
@@ -841,10 +882,11 @@ static hipError_t launch_advect_velocity(const Grid& g, const T* u0, const T* v0
                                          T* u1, T* v1, T* w1, const uint8_t* flags, float dt,
                                          hipStream_t st)
 {
-    const dim3 grid((unsigned)((g.nx - 1 + BX - 1) / BX), (unsigned)((g.ny - 1 + BY - 1) / BY),
-                    (unsigned)((g.nz - 1 + kAdvZC - 1) / kAdvZC));
+    dim3 grid((unsigned)((g.nx - 1 + BX - 1) / BX), (unsigned)((g.ny - 1 + BY - 1) / BY));
+    const int zc = advect_chunk(grid, g.nz - 1);
+    grid.z = (unsigned)((g.nz - 1 + zc - 1) / zc);
     hipLaunchKernelGGL(k_advect_velocity<T>, grid, dim3(BX, BY), 0, st, g, u0, v0, w0, u1, v1, w1,
-                       flags, dt);
+                       flags, dt, zc);
     return hipGetLastError();
 }
 hipError_t advect_velocity(const Grid& g, const float* u0, const float* v0, const float* w0,
@@ -858,10 +900,11 @@ template <typename T, typename TV>
 static hipError_t launch_advect_density(const Grid& g, const T* r0, T* r1, const TV* u, const TV* v,
                                         const TV* w, const uint8_t* flags, float dt, hipStream_t st)
 {
-    const dim3 grid((unsigned)((g.nx - 1 + BX - 1) / BX), (unsigned)((g.ny - 2 + BY - 1) / BY),
-                    (unsigned)((g.nz - 2 + kAdvZC - 1) / kAdvZC));
+    dim3 grid((unsigned)((g.nx - 1 + BX - 1) / BX), (unsigned)((g.ny - 2 + BY - 1) / BY));
+    const int zc = advect_chunk(grid, g.nz - 2);
+    grid.z = (unsigned)((g.nz - 2 + zc - 1) / zc);
     hipLaunchKernelGGL((k_advect_density<T, TV>), grid, dim3(BX, BY), 0, st, g, r0, r1, u, v, w,
-                       flags, dt);
+                       flags, dt, zc);
     return hipGetLastError();
 }
 hipError_t advect_density(const Grid& g, const float* r0, float* r1, const float* u,
@@ -905,10 +948,10 @@ hipError_t advect_density(const Grid& g, const float* r0, float* r1, const float
                            g.ny + 1, g.nz + 1);                                                    \
         return hipGetLastError();                                                                  \
     }                                                                                              \
-    hipError_t fill_source(const Grid& g, H* rho0, H* rho1, float4 sph, hipStream_t st,            \
-                           int* launched)                                                          \
+    hipError_t fill_sources(const Grid& g, H* rho0, H* rho1, const SphereList& src,                \
+                            hipStream_t st, int* launched)                                         \
     {                                                                                              \
-        return launch_source(g, rho0, rho1, sph, st, launched);                                    \
+        return launch_sources(g, rho0, rho1, src, st, launched);                                   \
     }                                                                                              \
     hipError_t force(const Grid& g, H* u, H* v, H* w, const H* rho, const uint8_t* flags,          \
                      const ForceArgs& a, hipStream_t st)                                           \
