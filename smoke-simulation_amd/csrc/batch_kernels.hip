@@ -147,16 +147,22 @@ __global__ __launch_bounds__(BX * BY) void kb_adv_d(const SimDesc* __restrict__ 
 }
 
 // Fused Jacobi sweeps over every tile of every simulation (TX x TY tiles,
-// R tile rows per thread).
+// R tile rows per thread).  One or two workgroups per CU walk blocks of very
+// different lengths (a chunk of the smallest and of the largest member), so
+// the launch lasts as long as the unluckiest workgroup: `order`, where there
+// is one, holds each workgroup's blocks so that all take about as long (the
+// starts of the gridDim.x lists and their end, then the lists; batch.cpp).
 template <int TX, int TY, int T, bool DAMPED, int R>
 __global__ __launch_bounds__(TX * TY / R, 8 / R) void kb_jacobi(const SimDesc* __restrict__ sims,
                                                      const StageTable* __restrict__ tab, int nsims,
-                                                     int lp, int zc, int zero_in, float omega)
+                                                     const int* __restrict__ order, int lp, int zc,
+                                                     int zero_in, float omega)
 {
     __shared__ dev::FusedLds<TX, TY, T> sh;
-    const int total = tab->start[nsims];
-    const VbRange r = vb_range(total);
-    for (int vb = r.begin; vb < r.end; vb += r.stride) {
+    VbRange r = vb_range(tab->start[nsims]);
+    if (order) r = {order[blockIdx.x], order[blockIdx.x + 1], 1};
+    for (int i = r.begin; i < r.end; i += r.stride) {
+        const int vb = order ? order[i] : i;
         const int si = find_owner(tab->start, nsims, vb);
         const int lb = vb - tab->start[si];
         const int gx = tab->gx[si], gy = tab->gy[si];
@@ -201,29 +207,29 @@ __global__ void kb_flip(SimDesc* __restrict__ sims, int nsims, int pflip)
 }
 
 template <int TX, int TY, int R, int T>
-hipError_t launch_bj(const SimDesc* sims, const StageTable* tab, int nsims, int grid, int lp,
-                     int zc, int zero_in, float omega, int plain, hipStream_t st)
+hipError_t launch_bj(const SimDesc* sims, const StageTable* tab, int nsims, const int* order,
+                     int grid, int lp, int zc, int zero_in, float omega, int plain, hipStream_t st)
 {
     const dim3 block(TX, TY / R);
     if (plain)
         hipLaunchKernelGGL((kb_jacobi<TX, TY, T, false, R>), dim3((unsigned)grid), block, 0, st,
-                           sims, tab, nsims, lp, zc, zero_in, omega);
+                           sims, tab, nsims, order, lp, zc, zero_in, omega);
     else
         hipLaunchKernelGGL((kb_jacobi<TX, TY, T, true, R>), dim3((unsigned)grid), block, 0, st,
-                           sims, tab, nsims, lp, zc, zero_in, omega);
+                           sims, tab, nsims, order, lp, zc, zero_in, omega);
     return hipGetLastError();
 }
 
 template <int TX, int TY, int R>
-hipError_t launch_bj_t(int t, const SimDesc* sims, const StageTable* tab, int nsims, int grid,
-                       int lp, int zc, int zero_in, float omega, int plain, hipStream_t st)
+hipError_t launch_bj_t(int t, const SimDesc* sims, const StageTable* tab, int nsims,
+                       const int* order, int grid, int lp, int zc, int zero_in, float omega, int plain, hipStream_t st)
 {
     switch (t) {
-    case 2: return launch_bj<TX, TY, R, 2>(sims, tab, nsims, grid, lp, zc, zero_in, omega, plain, st);
-    case 3: return launch_bj<TX, TY, R, 3>(sims, tab, nsims, grid, lp, zc, zero_in, omega, plain, st);
-    case 4: return launch_bj<TX, TY, R, 4>(sims, tab, nsims, grid, lp, zc, zero_in, omega, plain, st);
-    case 5: return launch_bj<TX, TY, R, 5>(sims, tab, nsims, grid, lp, zc, zero_in, omega, plain, st);
-    case 6: return launch_bj<TX, TY, R, 6>(sims, tab, nsims, grid, lp, zc, zero_in, omega, plain, st);
+    case 2: return launch_bj<TX, TY, R, 2>(sims, tab, nsims, order, grid, lp, zc, zero_in, omega, plain, st);
+    case 3: return launch_bj<TX, TY, R, 3>(sims, tab, nsims, order, grid, lp, zc, zero_in, omega, plain, st);
+    case 4: return launch_bj<TX, TY, R, 4>(sims, tab, nsims, order, grid, lp, zc, zero_in, omega, plain, st);
+    case 5: return launch_bj<TX, TY, R, 5>(sims, tab, nsims, order, grid, lp, zc, zero_in, omega, plain, st);
+    case 6: return launch_bj<TX, TY, R, 6>(sims, tab, nsims, order, grid, lp, zc, zero_in, omega, plain, st);
     default: return hipErrorInvalidValue;
     }
 }
@@ -276,7 +282,7 @@ hipError_t batch_cells(int stage, const SimDesc* sims, const StageTable* tab, in
 }
 
 hipError_t batch_jacobi(const SimDesc* sims, const StageTable* tab, int nsims, int total_blocks,
-                        int grid, const JacobiPlan& plan, int sweeps, int lp, int zero_in,
+                        const int* order, int grid, const JacobiPlan& plan, int sweeps, int lp, int zero_in,
                         float omega, int plain, hipStream_t st)
 {
     if (total_blocks <= 0) return hipSuccess;
@@ -288,17 +294,17 @@ hipError_t batch_jacobi(const SimDesc* sims, const StageTable* tab, int nsims, i
     if (plan.zc < 1) return hipErrorInvalidValue;
     switch (plan.tile) {
     case JacobiPlan::TILE_32x32:
-        return launch_bj_t<32, 32, 1>(sweeps, sims, tab, nsims, grid, lp, plan.zc, zero_in, omega,
-                                      plain, st);
+        return launch_bj_t<32, 32, 1>(sweeps, sims, tab, nsims, order, grid, lp, plan.zc, zero_in,
+                                      omega, plain, st);
     case JacobiPlan::TILE_64x16:
-        return launch_bj_t<64, 16, 1>(sweeps, sims, tab, nsims, grid, lp, plan.zc, zero_in, omega,
-                                      plain, st);
+        return launch_bj_t<64, 16, 1>(sweeps, sims, tab, nsims, order, grid, lp, plan.zc, zero_in,
+                                      omega, plain, st);
     case JacobiPlan::TILE_64x32:
-        return launch_bj_t<64, 32, 2>(sweeps, sims, tab, nsims, grid, lp, plan.zc, zero_in, omega,
-                                      plain, st);
+        return launch_bj_t<64, 32, 2>(sweeps, sims, tab, nsims, order, grid, lp, plan.zc, zero_in,
+                                      omega, plain, st);
     case JacobiPlan::TILE_32x64:
-        return launch_bj_t<32, 64, 2>(sweeps, sims, tab, nsims, grid, lp, plan.zc, zero_in, omega,
-                                      plain, st);
+        return launch_bj_t<32, 64, 2>(sweeps, sims, tab, nsims, order, grid, lp, plan.zc, zero_in,
+                                      omega, plain, st);
     default: return hipErrorInvalidValue;
     }
 }
@@ -331,6 +337,14 @@ hipError_t batch_advect_density(const SimDesc* sims, const StageTable* tab, int 
 }
 
 int batch_advect_density_blocks_per_cu() { return occupancy(kb_adv_d, BX * BY); }
+
+int batch_jacobi_block_steps(int sweeps, int planes)
+{
+    // The plane loop's trip count, and about 5 planes' time to start a block
+    // (table, first loads).
+    const int u = dev::z_unroll(sweeps);
+    return (planes + 2 * sweeps + u - 1) / u * u + 5;
+}
 
 int batch_jacobi_blocks_per_cu(const JacobiPlan& plan, int sweeps)
 {

@@ -199,8 +199,10 @@ hipError_t batch_sources(const SimDesc* sims, const SourceTable* tab, int total_
                          hipStream_t st);
 hipError_t batch_cells(int stage, const SimDesc* sims, const StageTable* tab, int nsims,
                        int total_blocks, int grid, int lp, hipStream_t st);
+// `order` (may be null, and is not used for single sweeps): the workgroups'
+// lists of blocks, for exactly `grid` workgroups (kb_jacobi).
 hipError_t batch_jacobi(const SimDesc* sims, const StageTable* tab, int nsims, int total_blocks,
-                        int grid, const JacobiPlan& plan, int sweeps, int lp, int zero_in,
+                        const int* order, int grid, const JacobiPlan& plan, int sweeps, int lp, int zero_in,
                         float omega, int plain, hipStream_t st);
 hipError_t batch_flip(SimDesc* sims, int nsims, int pflip, hipStream_t st);
 // Resident blocks per CU of the batched kernels (for sizing persistent grids).
@@ -216,6 +218,8 @@ hipError_t batch_advect_density(const SimDesc* sims, const StageTable* tab, int 
                                 int total_blocks, int grid, hipStream_t st);
 int batch_advect_density_blocks_per_cu();
 int batch_jacobi_blocks_per_cu(const JacobiPlan& plan, int sweeps);
+// Time of a block of `planes` planes, in planes marched (for balancing).
+int batch_jacobi_block_steps(int sweeps, int planes);
 
 // ------------------------------------------------------------ launchers
 // Every launcher enqueues on `st` and returns hipGetLastError().

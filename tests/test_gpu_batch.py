@@ -75,6 +75,27 @@ def test_batch_plans(plan):
         assert_bitwise_equal(st, o.state(), f"{sc['name']} plan {plan}")
 
 
+@pytest.mark.parametrize("dims,plan", [
+    ([(60, 200, 200), (57, 190, 180)], (6, 1, 1)),   # > 64 blocks per workgroup: by stride
+    ([(60, 70, 90), (9, 8, 12)], (3, 0, 2)),         # lists, the blocks' costs alike
+    ([(33, 30, 120), (120, 9, 7), (6, 6, 6)], (5, 2, 40)),  # lists, some of them empty
+])
+def test_batch_block_orders(dims, plan):
+    t, tile, zc = plan
+    scs = [scenes.test_scene(d, seed=60 + k, projection=smokesim.PROJ_JACOBI, iterations=t + 2,
+                             n_sources=1, n_obstacles=1) for k, d in enumerate(dims)]
+    sims = [gpu_for(sc) for sc in scs]
+    with smokesim.Batch(sims, [sc["dt"] for sc in scs]) as b:
+        b.set_jacobi_plan(sweeps_per_launch=t, tile=tile, zc=zc)
+        b.step(use_graph=False)
+        b.synchronize()
+        states = [s.state() for s in sims]
+    for sc, st in zip(scs, states):
+        o = oracle_for(sc, 32)
+        o.step(sc["dt"], 1)
+        assert_bitwise_equal(st, o.state(), f"{sc['name']} plan {plan}")
+
+
 def test_batch_autotune_and_readback():
     scs = members(iterations=9)
     sims = [gpu_for(sc) for sc in scs]
