@@ -290,7 +290,7 @@ struct HalfLds {
 // owning a pair of adjacent columns (x0, x0+1), x0 even, in R adjacent tile
 // rows.  The grown tile is 2*TXP cells wide and TY rows high; the inner
 // 2*TXP - 2T columns and TY - 2T rows are written (T even, so the inner
-// region is whole pairs).  Pairs cover x in [0, px): the cells beyond the
+// region is whole pairs).  Pairs cover x in [0, nx): the cells beyond the
 // interior have inv = 0 and r = 0, so they stay e = 0.  The diagonal inverse
 // of a cell is the FP16 rounding of cell_inv(flags byte), from a 256-entry
 // LDS table: the lane loads its pair's two flags bytes (one byte per cell
@@ -385,9 +385,13 @@ __device__ __forceinline__ void ref_sweep_levels(const Grid& g, const uint32_t* 
     };
 #pragma unroll
     for (int i = 0; i < D; ++i) load(z0 - T + i, i);
-    // Unrolled by lcm(3, T+1) so the register windows rotate without copies;
-    // the padded iterations load and write nothing.
-    constexpr int U = dev::z_unroll(T);
+    // Unrolled by a multiple of the windows' period of 3; the padded iterations
+    // load and write nothing.  The period of all rings (15 for T = 4, 21 for
+    // 6) would need no copies, but pads more and spills registers: 512^3, 18
+    // launches of 6 sweeps and two residuals 9.98 -> 9.84 ms a step, of 4 with
+    // two rows 13.9 -> 11.9; 120x111x130 (4 sweeps) 0.492 -> 0.401.  T = 4 has
+    // the registers for its five-deep rings to rotate in six.
+    constexpr int U = T == 4 ? 6 : 3;
     const int kend = z0 - T + ((z1 - z0 + 2 * T + U - 1) / U) * U;
     for (int kb = z0 - T; kb < kend; kb += U)
 #pragma unroll
@@ -445,11 +449,13 @@ __device__ __forceinline__ void ref_sweep_levels(const Grid& g, const uint32_t* 
                                       : __builtin_bit_cast(h2, sh.v[t - 1][prev][r0][tx + 1]);
                 const h2 Dp = (j + 1 < R) ? w[j + 1 < R ? j + 1 : 0][t - 1][1]
                                           : __builtin_bit_cast(h2, sh.v[t - 1][prev][r0 + R + 1][tx + 1]);
-                const h2 xm = {Lp.y, C.x};
-                const h2 xp = {C.y, Rp.x};
+                // {left + right} of both cells as one add: {Lp.y, Rp.x} with C's
+                // halves swapped (an operand selection, no instruction).
+                const h2 out = {Lp.y, Rp.x};
+                const h2 in = {C.y, C.x};
                 // Tree order, the z+ value (level t-1 of this iteration) last:
                 // the chain through the levels is one add and one fma per level.
-                const h2 part = ((xm + xp) + (Up + Dp)) + w[j][t - 1][0];
+                const h2 part = ((out + in) + (Up + Dp)) + w[j][t - 1][0];
                 const h2 sum = part + w[j][t - 1][2];
                 newv[j][t] = __builtin_elementwise_fma(iq[j][t], sum, -qq[j][t]);
             }
@@ -572,7 +578,8 @@ hipError_t reduce_and_finish(const RefineBufs& b, int n, int stage, double tol, 
 }
 
 // Tiles of 32 column pairs x 32 rows, one row per thread, or x 64 rows, two
-// rows per thread (1024 threads either way).
+// rows per thread (1024 threads either way).  In x the tiles cover the grid's
+// cells; the padding past them keeps the zeros it was created with.
 template <int T, bool FIRST, int R>
 hipError_t launch_sweeps(const Grid& g, const RefineBufs& b, const float* q, const uint8_t* flags,
                          int ein, int eout, int zc, hipStream_t st)
@@ -581,7 +588,7 @@ hipError_t launch_sweeps(const Grid& g, const RefineBufs& b, const float* q, con
     const uint16_t* flags2 = reinterpret_cast<const uint16_t*>(flags);
     constexpr int TXP = 32, TY = 32 * R;
     constexpr int OXC = 2 * TXP - 2 * T, OY = TY - 2 * T;
-    dim3 grid((unsigned)((g.px + OXC - 1) / OXC), (unsigned)((g.ny - 2 + OY - 1) / OY),
+    dim3 grid((unsigned)((g.nx + OXC - 1) / OXC), (unsigned)((g.ny - 2 + OY - 1) / OY),
               (unsigned)((g.nz - 2 + zc - 1) / zc));
     hipLaunchKernelGGL((k_ref_sweeps<TXP, TY, T, FIRST, R>), grid, dim3(TXP, TY / R), 0, st, g,
                        (const uint32_t*)b.e[ein], b.e[eout], q, b.qi, flags2, b.ctl,

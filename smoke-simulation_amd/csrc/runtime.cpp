@@ -1351,7 +1351,7 @@ smoke_status smoke_autotune(smoke_sim* s, smoke_jacobi_plan* chosen, double* ms_
             std::vector<int> lengths = zcs;
             const int w = refined ? 64 : smk::tile_width(tile), h = refined ? (tile == tiles[0] ? 32 : 64)
                                                                             : smk::tile_height(tile);
-            const int columns = ((refined ? s->g.px : s->g.nx - 2) + w - 2 * t - 1) / (w - 2 * t) *
+            const int columns = ((refined ? s->g.nx : s->g.nx - 2) + w - 2 * t - 1) / (w - 2 * t) *
                                 ((s->g.ny - 2 + h - 2 * t - 1) / (h - 2 * t));
             for (int per_cu = 1; per_cu <= 2; ++per_cu) {
                 const int chunks = std::max(1, per_cu * smk::kCUs / columns);

@@ -782,8 +782,8 @@ JacobiPlan fitted_plan(const Grid& g, bool refined)
     if (refined) {
         // FP16 pairs: 64x32-cell tiles (two per CU) of 4 sweeps, as unset plans had.
         constexpr int T = 4;
-        const ChunkModel half{2 * T, 15, 2, 0.45, 0.70};
-        plan.zc = fit_chunk(half, columns(g.px, m[1], 64 - 2 * T, 32 - 2 * T), m[2], std::min(64, most), &us);
+        const ChunkModel half{2 * T, 6, 2, 0.45, 0.70};
+        plan.zc = fit_chunk(half, columns(g.nx, m[1], 64 - 2 * T, 32 - 2 * T), m[2], std::min(64, most), &us);
         return plan;
     }
     constexpr int T = 5;
