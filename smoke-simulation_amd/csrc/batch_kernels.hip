@@ -104,7 +104,7 @@ __global__ __launch_bounds__(BX * BY) void kb_cells(const SimDesc* __restrict__ 
 // planes); the barrier after a column keeps the next column's ring stores
 // from overwriting planes still being read.  Every thread of a workgroup
 // walks the same columns.
-__global__ __launch_bounds__(BX * BY) void kb_adv_v(const SimDesc* __restrict__ sims,
+__global__ __launch_bounds__(BX * BY, 8) void kb_adv_v(const SimDesc* __restrict__ sims,
                                                     const StageTable* __restrict__ tab, int nsims)
 {
     __shared__ dev::AdvRing<BX, BY, 4, 3> ring;

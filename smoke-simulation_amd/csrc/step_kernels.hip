@@ -389,7 +389,7 @@ __global__ void k_gradient(Grid g, T* __restrict__ u, T* __restrict__ v, T* __re
 // Velocity advection: a block of BX x BY threads marches a column of BX x BY
 // cells through zc planes (dev::advect_velocity_march), in XCD tile order.
 template <typename T>
-__global__ __launch_bounds__(BX * BY) void k_advect_velocity(
+__global__ __launch_bounds__(BX * BY, 8) void k_advect_velocity(
     Grid g, const T* __restrict__ u0, const T* __restrict__ v0, const T* __restrict__ w0,
     T* __restrict__ u1, T* __restrict__ v1, T* __restrict__ w1, const uint8_t* __restrict__ flags,
     float dt, int zc)
@@ -404,7 +404,7 @@ __global__ __launch_bounds__(BX * BY) void k_advect_velocity(
 // Density advection: a block of BX x BY threads marches a column of BX x BY
 // cells through zc planes (dev::advect_density_march), in XCD tile order.
 template <typename T, typename TV>
-__global__ __launch_bounds__(BX * BY) void k_advect_density(
+__global__ __launch_bounds__(BX * BY, sizeof(T) == 2 ? 8 : 1) void k_advect_density(
     Grid g, const T* __restrict__ r0, T* __restrict__ r1, const TV* __restrict__ u,
     const TV* __restrict__ v, const TV* __restrict__ w, const uint8_t* __restrict__ flags, float dt,
     int zc)
