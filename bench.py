@@ -45,7 +45,7 @@ BYTES_SWEEP = 13               # P, d, flags in; P out
 BYTES_GRADIENT = 29            # P, u, v, w, flags in; u, v, w out
 BYTES_ADVECT_VEL = 25          # u, v, w, flags in; u, v, w out
 BYTES_ADVECT_DENS = 21         # rho, u, v, w, flags in; rho out
-BYTES_REF_HALF = 25            # in-place half-sweep on faces: u, v, w, flags in; u, v, w out
+BYTES_REF_HALF = 25            # half-sweeps of one launch on faces: u, v, w, flags in; u, v, w out
 BYTES_FIXED = (BYTES_FORCE + BYTES_DIVERGENCE + BYTES_GRADIENT + BYTES_ADVECT_VEL
                + BYTES_ADVECT_DENS)     # 121
 METRIC = "grid cell-updates/s per full step"
@@ -95,8 +95,8 @@ def step_bytes_per_cell(params, storage=0):
     if storage != 0:
         return fixed + BYTES_SWEEP * (k if params["projection"] == 2 else 2 * k)
     if params["projection"] == 0:
-        # In-place red-black half-sweep on faces: every u, v, w face is read
-        # and written once per half-sweep, plus the flags byte.
+        # Red-black half-sweep on faces, one per launch: every u, v, w face is
+        # read and written once per half-sweep, plus the flags byte.
         return BYTES_FORCE + BYTES_ADVECT_VEL + BYTES_ADVECT_DENS + 2 * k * BYTES_REF_HALF
     sweeps = k if params["projection"] == 2 else 2 * k
     return BYTES_FIXED + BYTES_SWEEP * sweeps
@@ -445,11 +445,14 @@ def run_single(args, sc):
             unfused = comp * sweeps_per_launch
             kernel = "k_jacobi_fused"
         elif p["projection"] == 1:
-            comp = unfused = BYTES_SWEEP * interior
-            kernel = "k_rbsor_half"
+            # Several half-sweeps per launch, 13 B per cell each launch.
+            comp = BYTES_SWEEP * interior
+            unfused = comp * 2 * p["iterations"] / launches_per_step
+            kernel = "k_ref_pressure_march"
         else:
-            comp = unfused = BYTES_REF_HALF * interior
-            kernel = "k_project_ref_half"
+            comp = BYTES_REF_HALF * interior
+            unfused = comp * 2 * p["iterations"] / launches_per_step
+            kernel = "k_ref_faces"
         achieved = comp / (avg_ms * 1e-3) / 1e9
         roofline = {
             "bound": "hbm", "kernel": kernel, "achieved": round(achieved, 1),
@@ -465,7 +468,7 @@ def run_single(args, sc):
             "sweeps_per_launch": sweeps_per_launch,
             "effective": {"bytes_per_launch": int(unfused),
                           "frac": round(unfused / (avg_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
-                          "model": "unfused: 13 B x interior cells x sweeps per launch"},
+                          "model": "unfused: the launch's bytes x its sweeps (half-sweeps)"},
             "launches_timed": r["sweep_launches"],
             "jacobi_plan": r["plan"] if p["projection"] in (2, 3) else None,
             "autotune": r["autotune"],
@@ -488,8 +491,11 @@ def run_single(args, sc):
     # Whole step: compulsory bytes with the launches the step makes (fixed
     # stages once, one sweep's 13 B per fused launch) and the unfused model.
     fixed = FIXED_BY_STORAGE[storage]
-    if p["projection"] == 2:
+    if p["projection"] in (1, 2):
         comp_bpc = fixed + BYTES_SWEEP * launches_per_step
+    elif p["projection"] == 0 and storage == 0:
+        comp_bpc = (BYTES_FORCE + BYTES_ADVECT_VEL + BYTES_ADVECT_DENS
+                    + BYTES_REF_HALF * launches_per_step)
     elif p["projection"] == 3:
         # Fused FP16 launches move the sweep bytes once each.
         refinements = -(-p["iterations"] // p["inner_sweeps"])
