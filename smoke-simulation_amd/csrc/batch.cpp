@@ -154,7 +154,9 @@ hipError_t upload_tables(smoke_batch* b)
 // 32..160 cells a side, 5 sweeps: 236 us (chunks of 64 planes) against 266 by
 // stride (chunks of 32; 280 with 64), a step of 60 sweeps 4.69 ms against 5.07.
 // The more blocks a workgroup has the less there is to balance: 14 each 319
-// and 326 us, 55 each 732 and 728; above 64 no lists are built.
+// and 326 us, 55 each 732 and 728; above 64 no lists are built.  With one block
+// per workgroup there is nothing to share, and walking a list costs a launch
+// about 1 us (two volumes of 18..98 a side, 90 launches: 3.00 -> 3.11 ms).
 void order_blocks(smoke_batch* b, int grid, std::vector<int>* out)
 {
     const smk::StageTable& t = b->h_tab[kTabJacobi];
@@ -205,7 +207,7 @@ hipError_t rebuild_jacobi_table(smoke_batch* b)
     b->order_grid = 0;
     const int t = b->plan.sweeps_per_launch, total = b->totals[kTabJacobi];
     const int grid = persistent_grid(b->occ_jacobi[t], b->cus, total);
-    if (e != hipSuccess || t < 2 || total > 64 * grid) return e;
+    if (e != hipSuccess || t < 2 || total <= grid || total > 64 * grid) return e;
     std::vector<int> order;
     order_blocks(b, grid, &order);
     if (order.size() > b->order_cap) {
