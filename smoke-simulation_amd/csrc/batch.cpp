@@ -43,6 +43,9 @@ struct smoke_batch {
     float omega = 1.0f;
     int plain = 1;
     smk::JacobiPlan plan;
+    // What smoke_batch_get_jacobi_plan reports: the first member's plan until
+    // one is set or tuned, though a batch of members without one runs fitted.
+    smk::JacobiPlan reported;
     long long cells = 0;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
@@ -195,6 +198,45 @@ void order_blocks(smoke_batch* b, int grid, std::vector<int>* out)
     out->assign(1, grid + 1);
     for (const std::vector<int>& l : lists) out->push_back(out->back() + (int)l.size());
     for (const std::vector<int>& l : lists) out->insert(out->end(), l.begin(), l.end());
+}
+
+// The plan of a batch whose members were never given one: 5 sweeps in the tile
+// and chunk with the least time by the step times of fitted_plan
+// (step_kernels.hip), the blocks taken as evenly shared.  With the members'
+// own 32x32 tiles of 64 planes a small batch occupies a few CUs: two volumes of
+// 18..98 a side, six steps of 60 sweeps 3.00 -> 1.36 ms.
+void fit_plan(smoke_batch* b)
+{
+    struct { int tile, per_cu; double one, full; } const tiles[2] = {
+        {smk::JacobiPlan::TILE_32x32, 2, 0.42, 0.66}, {smk::JacobiPlan::TILE_64x32, 1, 0.72, 0.73}};
+    smk::JacobiPlan best = b->plan;
+    double best_us = -1.0;
+    for (const auto& t : tiles)
+        for (int zc = 8; zc <= 256; zc *= 2) {
+            b->plan.sweeps_per_launch = 5;
+            b->plan.tile = t.tile;
+            b->plan.zc = std::min(zc, b->zc_cap);
+            smk::StageTable tab;
+            int total = 0, longest = 0;
+            fill_table(tab, b->sims, kTabJacobi, b->plan, &total);
+            double steps = 0.0;
+            for (size_t s = 0; s < b->sims.size(); ++s) {
+                const int columns = tab.gx[s] * tab.gy[s];
+                for (int z = 0, n = b->sims[s]->g.nz - 2; z < n; z += b->plan.zc) {
+                    const int c = smk::batch_jacobi_block_steps(5, std::min(b->plan.zc, n - z));
+                    steps += (double)columns * c;
+                    longest = std::max(longest, c);
+                }
+            }
+            const double us = total <= b->cus
+                                  ? longest * t.one
+                                  : std::max((double)longest, steps / (t.per_cu * b->cus)) * t.full;
+            if (best_us < 0.0 || us < best_us) {
+                best_us = us;
+                best = b->plan;
+            }
+        }
+    b->plan = best;
 }
 
 // The plan's table and block order.  The stream must be idle.
@@ -363,6 +405,7 @@ smoke_status smoke_batch_create(smoke_sim* const* sims, int count, const float* 
     for (int i = 0; i < count; ++i) b->zc_cap = std::min(b->zc_cap, smk::fused_max_zc(sims[i]->g.plane));
     b->plan = sims[0]->plan;
     b->plan.zc = std::min(b->plan.zc, b->zc_cap);
+    b->reported = b->plan;
     auto bail = [&](smoke_status st) {
         smoke_batch_destroy(b);
         return st;
@@ -370,6 +413,7 @@ smoke_status smoke_batch_create(smoke_sim* const* sims, int count, const float* 
     hipDeviceProp_t prop;
     if (hipGetDeviceProperties(&prop, dev) != hipSuccess) return bail(fail(SMOKE_ERR_HIP, "batch_create: device query"));
     b->cus = prop.multiProcessorCount;
+    if (!sims[0]->plan_set) fit_plan(b);
     if (hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) != hipSuccess)
         return bail(fail(SMOKE_ERR_HIP, "batch_create: stream"));
     // Freeze the scene: masks up to date, all earlier work on the
@@ -545,6 +589,7 @@ smoke_status smoke_batch_set_jacobi_plan(smoke_batch* b, const smoke_jacobi_plan
     b->plan.sweeps_per_launch = plan->sweeps_per_launch;
     b->plan.tile = plan->tile;
     b->plan.zc = std::min(plan->zc, b->zc_cap);
+    b->reported = b->plan;
     drop_graph(b);
     HIP_TRY(rebuild_jacobi_table(b));
     return SMOKE_OK;
@@ -553,9 +598,9 @@ smoke_status smoke_batch_set_jacobi_plan(smoke_batch* b, const smoke_jacobi_plan
 smoke_status smoke_batch_get_jacobi_plan(const smoke_batch* b, smoke_jacobi_plan* out)
 {
     if (!b || !out) return fail(SMOKE_ERR_INVALID, "batch_get_jacobi_plan: NULL");
-    out->sweeps_per_launch = b->plan.sweeps_per_launch;
-    out->tile = b->plan.tile;
-    out->zc = b->plan.zc;
+    out->sweeps_per_launch = b->reported.sweeps_per_launch;
+    out->tile = b->reported.tile;
+    out->zc = b->reported.zc;
     return SMOKE_OK;
 }
 
@@ -599,7 +644,7 @@ smoke_status smoke_batch_autotune(smoke_batch* b, smoke_jacobi_plan* chosen, dou
             }
     (void)hipEventDestroy(ev[0]);
     (void)hipEventDestroy(ev[1]);
-    b->plan = best;
+    b->plan = b->reported = best;
     if (e == hipSuccess) e = rebuild_jacobi_table(b);
     if (e != hipSuccess) return fail(SMOKE_ERR_HIP, "batch_autotune: %s", hipGetErrorString(e));
     if (chosen) {

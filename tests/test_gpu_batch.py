@@ -96,6 +96,23 @@ def test_batch_block_orders(dims, plan):
         assert_bitwise_equal(st, o.state(), f"{sc['name']} plan {plan}")
 
 
+@pytest.mark.parametrize("given", [None, dict(sweeps_per_launch=3, tile=1, zc=7)])
+def test_batch_plan_of_its_first_member(given):
+    scs = members(iterations=13)
+    sims = [gpu_for(sc) for sc in scs]
+    if given:
+        sims[0].set_jacobi_plan(**given)
+    with smokesim.Batch(sims, [sc["dt"] for sc in scs]) as b:
+        assert b.get_jacobi_plan() == (given or dict(sweeps_per_launch=4, tile=0, zc=64))
+        b.step(use_graph=True)
+        b.synchronize()
+        states = [s.state() for s in sims]
+    for sc, st in zip(scs, states):
+        o = oracle_for(sc, 32)
+        o.step(sc["dt"], 1)
+        assert_bitwise_equal(st, o.state(), f"{sc['name']} plan {given}")
+
+
 def test_batch_autotune_and_readback():
     scs = members(iterations=9)
     sims = [gpu_for(sc) for sc in scs]
