@@ -746,18 +746,16 @@ bool bounce_ready(Bounce& b, int device)
     return true;
 }
 
-// Host memory the DMA engines reach directly (hipHostMalloc, registered).
-// The symbol is missing where no GPU runtime is linked.
-#pragma weak hipPointerGetAttributes
-bool pinned(const void* p)
+// Plain host memory, unknown to the GPU runtime.  Any other target (pinned,
+// registered or managed memory, device memory) is the runtime's to write: the
+// CPU may not even be able to.
+bool pageable(const void* p)
 {
-    if (!&hipPointerGetAttributes) return false;
     hipPointerAttribute_t a;
-    if (hipPointerGetAttributes(&a, p) != hipSuccess) {
-        smk::forget_last_error();
-        return false;
-    }
-    return a.type == hipMemoryTypeHost;
+    const hipError_t e = hipPointerGetAttributes(&a, p);
+    if (e == hipSuccess) return a.type == hipMemoryTypeUnregistered;
+    smk::forget_last_error();
+    return e == hipErrorInvalidValue;  // as some runtimes answer for such memory
 }
 
 // Copies `bytes` of device memory to host memory after the work on the
@@ -770,7 +768,7 @@ smoke_status copy_to_host(smoke_sim* s, void* dst, const void* dev, size_t bytes
 {
     std::unique_lock<std::mutex> lk(g_bounce.mu, std::defer_lock);
     int device = -1;
-    if (bytes < (64u << 10) || pinned(dst) || hipGetDevice(&device) != hipSuccess ||
+    if (bytes < (64u << 10) || !pageable(dst) || hipGetDevice(&device) != hipSuccess ||
         device != s->device || !lk.try_lock() || !bounce_ready(g_bounce, device)) {
         HIP_TRY(hipMemcpyAsync(dst, dev, bytes, hipMemcpyDeviceToHost, s->stream));
         HIP_TRY(hipStreamSynchronize(s->stream));

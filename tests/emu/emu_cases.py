@@ -321,7 +321,48 @@ def case_norms():
     g.close()
 
 
-CASES = {"step_graph": case_step_graph, "proxy": case_proxy, "refine_groups": case_refine_groups, "single": case_single, "norms": case_norms, "plans": case_plans, "batch": case_batch,
+class EmuDevice:
+    """Device memory of the emulator, as a caller of the C ABI holds it."""
+
+    def __init__(self, nbytes):
+        import ctypes
+        self.lib = smokesim.load()
+        self.lib.emu_copies_into.restype = ctypes.c_longlong
+        self.lib.emu_copies_into.argtypes = [ctypes.c_void_p]
+        self.lib.hipFree.argtypes = [ctypes.c_void_p]
+        p = ctypes.c_void_p()
+        assert self.lib.hipMalloc(ctypes.byref(p), ctypes.c_size_t(nbytes)) == 0
+        self.p = p
+        self.floats = np.ctypeslib.as_array(ctypes.cast(p, ctypes.POINTER(ctypes.c_float)), (nbytes // 4,))
+
+    def copies(self):
+        return self.lib.emu_copies_into(self.p)
+
+    def free(self):
+        del self.floats
+        assert self.lib.hipFree(self.p) == 0
+
+
+def case_read_targets():
+    # A blocking read into device memory is one copy by the runtime, whatever
+    # its size and whatever reads into host memory came before; only plain host
+    # memory is written by the CPU.
+    import ctypes
+    rng = np.random.default_rng(11)
+    for dims in ((20, 17, 13), (40, 33, 30), (112, 100, 84)):  # 17 KB, 155 KB, 3.6 MB
+        x = rng.standard_normal(dims[::-1]).astype(np.float32)
+        g = smokesim.Simulation(*dims, density=x)
+        for _ in range(6):
+            same_bits(g.get_density(0), x, f"{dims} into host memory")
+        dev = EmuDevice(x.nbytes)
+        smokesim._check(g.lib.smoke_get_density(g.h, 0, ctypes.cast(dev.p, ctypes.POINTER(ctypes.c_float))))
+        assert dev.copies() == 1, (dims, dev.copies())
+        same_bits(dev.floats, x.ravel(), f"{dims} into device memory")
+        dev.free()
+        g.close()
+
+
+CASES = {"read_targets": case_read_targets, "step_graph": case_step_graph, "proxy": case_proxy, "refine_groups": case_refine_groups, "single": case_single, "norms": case_norms, "plans": case_plans, "batch": case_batch,
          "server": case_server, "readback": case_readback, "precision": case_precision,
          "vorticity": case_vorticity, "advection": case_advection}
 

@@ -24,6 +24,8 @@
 //    time, which is what makes `static` stand in for LDS.
 //  * Handles carry magic numbers and are checked on every use, so a call on
 //    a destroyed stream, event or graph stops the run.
+//  * Copies, event calls and allocations may come from several threads.
+//    emu_copies_into and the like below tell a test what was called.
 #include <hip/hip_runtime_api.h>
 
 #include <barrier>
@@ -35,8 +37,8 @@
 #include <algorithm>
 #include <deque>
 #include <functional>
+#include <map>
 #include <memory>
-#include <set>
 #include <thread>
 #include <vector>
 
@@ -74,7 +76,10 @@ thread_local EmuIdx threadIdx, blockIdx, blockDim, gridDim;
 
 namespace {
 
-std::set<void*> g_device;
+std::map<void*, size_t> g_device, g_pinned;  // base and size
+std::map<void*, long long> g_copies;         // by device allocation: copies into it
+std::recursive_mutex g_mu;                   // held by the calls several threads make
+using Lock = std::lock_guard<std::recursive_mutex>;
 const bool g_deferred = getenv("EMU_DEFERRED") != nullptr;
 const bool g_reverse_blocks = getenv("EMU_REVERSE_BLOCKS") != nullptr;
 ihipStream_t g_null_stream{0x5354524dU, false, {}, {}, 0, 0};
@@ -94,6 +99,14 @@ bool g_threaded = false;
 void check(hipStream_t s)
 {
     if (s && s->magic != kStream) die("use of an invalid stream");
+}
+// The allocation that holds p, or null.
+void* base_of(const std::map<void*, size_t>& m, const void* p)
+{
+    auto it = m.upper_bound(const_cast<void*>(p));
+    if (it == m.begin()) return nullptr;
+    --it;
+    return static_cast<const char*>(p) < static_cast<char*>(it->first) + it->second ? it->first : nullptr;
 }
 void check(hipEvent_t e)
 {
@@ -305,27 +318,43 @@ extern "C" {
 
 hipError_t hipMalloc(void** p, size_t n)
 {
+    Lock lk(g_mu);
     *p = malloc(n ? n : 1);
-    g_device.insert(*p);
+    g_device[*p] = n;
     return hipSuccess;
 }
 hipError_t hipFree(void* p)
 {
     if (!p) return hipSuccess;
+    Lock lk(g_mu);
     drain_all();
+    g_copies.erase(p);
     if (!g_device.erase(p)) die("hipFree of a pointer hipMalloc did not return");
     free(p);
     return hipSuccess;
 }
 hipError_t hipHostMalloc(void** p, size_t n, unsigned)
 {
+    Lock lk(g_mu);
     *p = malloc(n ? n : 1);
+    g_pinned[*p] = n;
     return hipSuccess;
 }
 hipError_t hipHostFree(void* p)
 {
+    Lock lk(g_mu);
     drain_all();
+    g_pinned.erase(p);
     free(p);
+    return hipSuccess;
+}
+hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void* p)
+{
+    Lock lk(g_mu);
+    memset(a, 0, sizeof *a);
+    a->type = base_of(g_device, p)   ? hipMemoryTypeDevice
+              : base_of(g_pinned, p) ? hipMemoryTypeHost
+                                     : hipMemoryTypeUnregistered;
     return hipSuccess;
 }
 hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind)
@@ -337,6 +366,8 @@ hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipSt
 {
     check(st);
     if (st && st->capturing) die("copy recorded into a graph");
+    Lock lk(g_mu);
+    if (void* base = base_of(g_device, d)) g_copies[base] += 1;
     enqueue(st, [=]() { memcpy(d, s, n); });
     return hipSuccess;
 }
@@ -386,6 +417,7 @@ hipError_t hipStreamDestroy(hipStream_t s)
 }
 hipError_t hipStreamSynchronize(hipStream_t s)
 {
+    Lock lk(g_mu);
     check(s);
     if (s && s->capturing) die("synchronize on a capturing stream");
     drain(S(s), S(s)->enqueued);
@@ -461,6 +493,7 @@ hipError_t hipEventDestroy(hipEvent_t e)
 }
 hipError_t hipEventRecord(hipEvent_t e, hipStream_t s)
 {
+    Lock lk(g_mu);
     check(e);
     check(s);
     if (s && s->capturing) return hipSuccess;  // not part of the recorded work
@@ -470,12 +503,14 @@ hipError_t hipEventRecord(hipEvent_t e, hipStream_t s)
 }
 hipError_t hipEventSynchronize(hipEvent_t e)
 {
+    Lock lk(g_mu);
     check(e);
     if (e->stream) drain(e->stream, e->target);
     return hipSuccess;
 }
 hipError_t hipEventQuery(hipEvent_t e)
 {
+    Lock lk(g_mu);
     check(e);
     return !e->stream || e->stream->done >= e->target ? hipSuccess : hipErrorNotReady;
 }
@@ -486,6 +521,14 @@ hipError_t hipEventElapsedTime(float* ms, hipEvent_t a, hipEvent_t b)
     if (hipEventQuery(a) != hipSuccess || hipEventQuery(b) != hipSuccess) return hipErrorNotReady;
     *ms = 1.0f;
     return hipSuccess;
+}
+
+// What a test asks of the emulator: the asynchronous copies into the device
+// allocation at `base` so far.
+long long emu_copies_into(void* base)
+{
+    Lock lk(g_mu);
+    return g_copies.count(base) ? g_copies[base] : 0;
 }
 
 }  // extern "C"

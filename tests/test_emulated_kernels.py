@@ -58,3 +58,15 @@ def test_emulated_case_with_deferred_streams(emu_lib, case):
     r = subprocess.run([sys.executable, os.path.join(EMU, "emu_cases.py"), lib, case], env=env,
                        capture_output=True, text=True, timeout=600)
     assert r.returncode == 0 and f"ok {case}" in r.stdout, (r.stdout[-4000:] + r.stderr[-8000:])
+
+
+@pytest.mark.parametrize("case,deferred", [("read_targets", False), ("read_targets", True)])
+def test_emulated_host_path(emu_lib, case, deferred):
+    """What the host code asks of the runtime (tests/emu/emu_cases.py)."""
+    lib, asan = emu_lib
+    env = dict(os.environ, LD_PRELOAD=asan, ASAN_OPTIONS="detect_leaks=0:abort_on_error=0")
+    if deferred:
+        env["EMU_DEFERRED"] = "1"
+    r = subprocess.run([sys.executable, os.path.join(EMU, "emu_cases.py"), lib, case], env=env,
+                       capture_output=True, text=True, timeout=600)
+    assert r.returncode == 0 and f"ok {case}" in r.stdout, (r.stdout[-4000:] + r.stderr[-8000:])
