@@ -251,12 +251,21 @@ smoke_status ensure_vort(smoke_sim* s)
     return SMOKE_OK;
 }
 
+// While it lives, this thread's allocations are allowed although some thread
+// captures a stream: in the default mode they fail then, and end the capture.
+struct AllowWhileCapturing {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    AllowWhileCapturing() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    ~AllowWhileCapturing() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
 // Allocates the reference projection's second velocity set (once per
-// simulation, before a step or a capture).  Its launches write every entry
-// they later read.
+// simulation, before a step or a capture of its own).  Its launches write
+// every entry they later read.
 void ensure_sweep_fields(smoke_sim* s)
 {
     if (s->prm.projection != SMOKE_PROJ_REFERENCE || s->sweep_mem || s->sweep_refused) return;
+    const AllowWhileCapturing allow;
     const size_t field = align256((size_t)s->g.elems * sizeof(float));
     if (hipMalloc((void**)&s->sweep_mem, 3 * field) != hipSuccess) {
         smk::forget_last_error();  // the launches' checks must not find it

@@ -362,7 +362,38 @@ def case_read_targets():
         g.close()
 
 
-CASES = {"read_targets": case_read_targets, "step_graph": case_step_graph, "proxy": case_proxy, "refine_groups": case_refine_groups, "single": case_single, "norms": case_norms, "plans": case_plans, "batch": case_batch,
+def _sweep_launches(g, dt):
+    """Launches of the projection's sweeps in one step."""
+    g.timing_enable(True)
+    g.timing_reset()
+    g.step(dt, readback=False)
+    n = g.timing_sweeps()[1]
+    g.timing_enable(False)
+    return n
+
+
+def case_foreign_capture():
+    # A first step of the reference form while another stream is captured in
+    # the global mode: the capture goes on, and this and later steps run
+    # several half-sweeps per launch.
+    import ctypes
+    sc = scenes.test_scene((14, 12, 10), seed=36, projection=0, iterations=6)
+    g, o = gpu_for(sc), oracle_for(sc, 32)
+    hip = smokesim.load()
+    st, graph = ctypes.c_void_p(), ctypes.c_void_p()
+    assert hip.hipStreamCreateWithFlags(ctypes.byref(st), 1) == 0
+    assert hip.hipStreamBeginCapture(st, 0) == 0
+    g.step(sc["dt"], readback=False)
+    assert hip.hipStreamEndCapture(st, ctypes.byref(graph)) == 0
+    assert hip.hipGraphDestroy(graph) == 0 and hip.hipStreamDestroy(st) == 0
+    n = _sweep_launches(g, sc["dt"])
+    assert n < 2 * 6, n
+    o.step(sc["dt"], 2)
+    assert_bitwise_equal(g.state(), o.state(), "foreign capture")
+    g.close()
+
+
+CASES = {"foreign_capture": case_foreign_capture, "read_targets": case_read_targets, "step_graph": case_step_graph, "proxy": case_proxy, "refine_groups": case_refine_groups, "single": case_single, "norms": case_norms, "plans": case_plans, "batch": case_batch,
          "server": case_server, "readback": case_readback, "precision": case_precision,
          "vorticity": case_vorticity, "advection": case_advection}
 

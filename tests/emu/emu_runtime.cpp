@@ -24,6 +24,8 @@
 //    time, which is what makes `static` stand in for LDS.
 //  * Handles carry magic numbers and are checked on every use, so a call on
 //    a destroyed stream, event or graph stops the run.
+//  * Allocations end the captures the runtime's rules protect: those in the
+//    global mode, unless the thread exchanged its own mode.
 //  * Copies, event calls and allocations may come from several threads.
 //    emu_copies_into and the like below tell a test what was called.
 #include <hip/hip_runtime_api.h>
@@ -54,6 +56,8 @@ struct ihipStream_t {
     std::vector<Op> rec;
     std::deque<Op> queue;  // deferred work not yet run
     unsigned long long enqueued = 0, done = 0;
+    hipStreamCaptureMode mode = hipStreamCaptureModeGlobal;  // of the capture
+    bool invalid = false;                                    // the capture was ended by a call
 };
 struct ihipEvent_t {
     unsigned magic;
@@ -82,7 +86,7 @@ std::recursive_mutex g_mu;                   // held by the calls several thread
 using Lock = std::lock_guard<std::recursive_mutex>;
 const bool g_deferred = getenv("EMU_DEFERRED") != nullptr;
 const bool g_reverse_blocks = getenv("EMU_REVERSE_BLOCKS") != nullptr;
-ihipStream_t g_null_stream{0x5354524dU, false, {}, {}, 0, 0};
+ihipStream_t g_null_stream{0x5354524dU, false, {}, {}};
 std::vector<ihipStream_t*> g_streams;  // live streams, in creation order (null stream first)
 std::barrier<>* g_barrier = nullptr;
 // One barrier per wave of 64 threads for lane exchanges (DPP, shuffles): a
@@ -99,6 +103,17 @@ bool g_threaded = false;
 void check(hipStream_t s)
 {
     if (s && s->magic != kStream) die("use of an invalid stream");
+}
+// A call that captures forbid: true, and the captures are ended, unless this
+// thread's mode allows it.
+thread_local hipStreamCaptureMode t_mode = hipStreamCaptureModeGlobal;
+bool unsafe_call()
+{
+    bool any = false;
+    for (ihipStream_t* s : g_streams)
+        if (t_mode == hipStreamCaptureModeGlobal && s->capturing && s->mode == hipStreamCaptureModeGlobal)
+            any = s->invalid = true;
+    return any;
 }
 // The allocation that holds p, or null.
 void* base_of(const std::map<void*, size_t>& m, const void* p)
@@ -319,6 +334,7 @@ extern "C" {
 hipError_t hipMalloc(void** p, size_t n)
 {
     Lock lk(g_mu);
+    if (unsafe_call()) return hipErrorStreamCaptureUnsupported;
     *p = malloc(n ? n : 1);
     g_device[*p] = n;
     return hipSuccess;
@@ -336,6 +352,7 @@ hipError_t hipFree(void* p)
 hipError_t hipHostMalloc(void** p, size_t n, unsigned)
 {
     Lock lk(g_mu);
+    if (unsafe_call()) return hipErrorStreamCaptureUnsupported;
     *p = malloc(n ? n : 1);
     g_pinned[*p] = n;
     return hipSuccess;
@@ -399,7 +416,7 @@ hipError_t hipGetDevicePropertiesR0600(hipDeviceProp_tR0600* p, int)
 const char* hipGetErrorString(hipError_t) { return "emulator error"; }
 hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned)
 {
-    *s = new ihipStream_t{kStream, false, {}, {}, 0, 0};
+    *s = new ihipStream_t{kStream, false, {}, {}};
     g_streams.push_back(*s);
     return hipSuccess;
 }
@@ -433,16 +450,28 @@ hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned)
     if (es) enqueue(s, [es, t]() { drain(es, t); });
     return hipSuccess;
 }
-hipError_t hipStreamBeginCapture(hipStream_t s, hipStreamCaptureMode)
+hipError_t hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode* mode)
+{
+    std::swap(*mode, t_mode);
+    return hipSuccess;
+}
+hipError_t hipStreamBeginCapture(hipStream_t s, hipStreamCaptureMode mode)
 {
     check(s);
     s->capturing = true;
+    s->mode = mode;
+    s->invalid = false;
     return hipSuccess;
 }
 hipError_t hipStreamEndCapture(hipStream_t s, hipGraph_t* g)
 {
     check(s);
     s->capturing = false;
+    if (s->invalid) {
+        s->rec.clear();
+        *g = nullptr;
+        return hipErrorStreamCaptureInvalidated;
+    }
     *g = new ihipGraph{kGraph, std::move(s->rec)};
     s->rec.clear();
     return hipSuccess;

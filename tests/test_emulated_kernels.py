@@ -60,7 +60,8 @@ def test_emulated_case_with_deferred_streams(emu_lib, case):
     assert r.returncode == 0 and f"ok {case}" in r.stdout, (r.stdout[-4000:] + r.stderr[-8000:])
 
 
-@pytest.mark.parametrize("case,deferred", [("read_targets", False), ("read_targets", True)])
+@pytest.mark.parametrize("case,deferred", [("read_targets", False), ("read_targets", True),
+                                           ("foreign_capture", False)])
 def test_emulated_host_path(emu_lib, case, deferred):
     """What the host code asks of the runtime (tests/emu/emu_cases.py)."""
     lib, asan = emu_lib
