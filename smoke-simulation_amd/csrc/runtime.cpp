@@ -770,14 +770,21 @@ bool pageable(const void* p)
 // Copies `bytes` of device memory to host memory after the work on the
 // simulation's stream, and waits for it.  The runtime's copy to pageable
 // memory moves it in turns, DMA then one thread's memcpy, and the caller's
-// pages are often new: 61 MB took 8 ms, 7.6 GB/s.  Here the pieces go through
+// pages are often new: 64 MB take 6.7 ms, 9.5 GB/s.  Here the pieces go through
 // pinned slots, one per thread (a thread for every 1 MB, at most 8), so that
-// DMA, memcpy and page faults of different pieces overlap.
+// DMA, memcpy and page faults of different pieces overlap: 2.0 ms.
+//
+// Reads below 4 MB take the runtime's copy: with slots they were no faster
+// where a wait for the GPU takes a few us (ms, runtime's / slots: 1 MB 0.08 /
+// 0.08, 2 MB 0.13 / 0.13, 4 MB 0.24 / 0.22, 5 MB 0.30 / 0.26, 8 MB 0.47 /
+// 0.38), and every piece is one more wait where it takes 0.1 ms (64 KB 0.03 /
+// 0.13, 1 MB 0.15 / 0.28, 2 MB 0.29 / 0.45, 3.5 MB 0.58 / 0.64).
+constexpr size_t kSlotReadBytes = 4u << 20;
 smoke_status copy_to_host(smoke_sim* s, void* dst, const void* dev, size_t bytes)
 {
     std::unique_lock<std::mutex> lk(g_bounce.mu, std::defer_lock);
     int device = -1;
-    if (bytes < (64u << 10) || !pageable(dst) || hipGetDevice(&device) != hipSuccess ||
+    if (bytes < kSlotReadBytes || !pageable(dst) || hipGetDevice(&device) != hipSuccess ||
         device != s->device || !lk.try_lock() || !bounce_ready(g_bounce, device)) {
         HIP_TRY(hipMemcpyAsync(dst, dev, bytes, hipMemcpyDeviceToHost, s->stream));
         HIP_TRY(hipStreamSynchronize(s->stream));
@@ -785,52 +792,32 @@ smoke_status copy_to_host(smoke_sim* s, void* dst, const void* dev, size_t bytes
     }
     char* const out = static_cast<char*>(dst);
     const char* const in = static_cast<const char*>(dev);
-    auto fetch = [&](int slot, char* b, size_t at, size_t n) {
-        const hipError_t e = hipMemcpyAsync(b, in + at, n, hipMemcpyDeviceToHost, s->stream);
-        return e == hipSuccess ? hipEventRecord(g_bounce.ev[slot], s->stream) : e;
-    };
-    auto finish = [&](int slot, const char* b, size_t at, size_t n) {
-        const hipError_t e = hipEventSynchronize(g_bounce.ev[slot]);
-        if (e == hipSuccess) std::memcpy(out + at, b, n);
-        return e;
-    };
-    // (Below 3 MB starting a thread costs as much as it saves.)
-    const int threads = bytes < (3u << 20) ? 1 : (int)std::min<size_t>(kBounceSlots, bytes >> 20);
+    const int threads = (int)std::min<size_t>(kBounceSlots, bytes >> 20);
+    const size_t width = std::min(kBounceBytes, (bytes / threads + 4095) / 4096 * 4096);
     std::atomic<int> failed{(int)hipSuccess};
-    if (threads <= 1) {
-        // One thread: every piece's DMA is enqueued, then each is copied out.
-        constexpr size_t kPiece = 512u << 10;
-        static_assert((3u << 20) <= kBounceSlots * kPiece, "a slot for every piece");
-        hipError_t e = hipSuccess;
-        for (size_t at = 0, k = 0; e == hipSuccess && at < bytes; at += kPiece, ++k)
-            e = fetch((int)k, g_bounce.mem + at, at, std::min(kPiece, bytes - at));
-        for (size_t at = 0, k = 0; e == hipSuccess && at < bytes; at += kPiece, ++k)
-            e = finish((int)k, g_bounce.mem + at, at, std::min(kPiece, bytes - at));
-        failed = (int)e;
-    } else {
-        const size_t width = std::min(kBounceBytes, (bytes / threads + 4095) / 4096 * 4096);
-        auto run = [&](int slot, bool helper) {
-            hipError_t e = helper ? hipSetDevice(device) : hipSuccess;
-            char* const b = g_bounce.mem + slot * kBounceBytes;
-            for (size_t at = slot * width; e == hipSuccess && at < bytes; at += threads * width) {
-                const size_t n = std::min(width, bytes - at);
-                e = fetch(slot, b, at, n);
-                if (e == hipSuccess) e = finish(slot, b, at, n);
-            }
-            if (e != hipSuccess) failed = (int)e;
-        };
-        std::vector<std::thread> helpers;
-        try {
-            helpers.reserve((size_t)threads);
-            for (int k = 1; k < threads; ++k) helpers.emplace_back(run, k, true);
-        } catch (const std::exception&) {
-            // The pieces of a thread that could not start are copied below.
+    auto run = [&](int slot, bool helper) {
+        hipError_t e = helper ? hipSetDevice(device) : hipSuccess;
+        char* const b = g_bounce.mem + slot * kBounceBytes;
+        for (size_t at = slot * width; e == hipSuccess && at < bytes; at += threads * width) {
+            const size_t n = std::min(width, bytes - at);
+            e = hipMemcpyAsync(b, in + at, n, hipMemcpyDeviceToHost, s->stream);
+            if (e == hipSuccess) e = hipEventRecord(g_bounce.ev[slot], s->stream);
+            if (e == hipSuccess) e = hipEventSynchronize(g_bounce.ev[slot]);
+            if (e == hipSuccess) std::memcpy(out + at, b, n);
         }
-        const int started = (int)helpers.size() + 1;
-        run(0, false);
-        for (int k = started; k < threads; ++k) run(k, false);
-        for (std::thread& t : helpers) t.join();
+        if (e != hipSuccess) failed = (int)e;
+    };
+    std::vector<std::thread> helpers;
+    try {
+        helpers.reserve((size_t)threads);
+        for (int k = 1; k < threads; ++k) helpers.emplace_back(run, k, true);
+    } catch (const std::exception&) {
+        // The pieces of a thread that could not start are copied below.
     }
+    const int started = (int)helpers.size() + 1;
+    run(0, false);
+    for (int k = started; k < threads; ++k) run(k, false);
+    for (std::thread& t : helpers) t.join();
     const hipError_t done = hipStreamSynchronize(s->stream);  // no copy still writes a slot
     HIP_TRY((hipError_t)failed.load());
     HIP_TRY(done);

@@ -349,7 +349,7 @@ def case_read_targets():
     # memory is written by the CPU.
     import ctypes
     rng = np.random.default_rng(11)
-    for dims in ((20, 17, 13), (40, 33, 30), (112, 100, 84)):  # 17 KB, 155 KB, 3.6 MB
+    for dims in ((20, 17, 13), (40, 33, 30), (120, 100, 91)):  # 17 KB, 155 KB, 4.2 MB
         x = rng.standard_normal(dims[::-1]).astype(np.float32)
         g = smokesim.Simulation(*dims, density=x)
         for _ in range(6):
@@ -360,6 +360,24 @@ def case_read_targets():
         same_bits(dev.floats, x.ravel(), f"{dims} into device memory")
         dev.free()
         g.close()
+
+
+def _pinned_calls():
+    import ctypes
+    f = smokesim.load().emu_pinned_calls
+    f.restype = ctypes.c_longlong
+    return f()
+
+
+def case_small_reads():
+    # Reads below 4 MB are the runtime's copies: no pinned pieces.
+    rng = np.random.default_rng(12)
+    for dims in ((40, 33, 30), (101, 100, 99)):  # 155 KB, 3.8 MB
+        x = rng.standard_normal(dims[::-1]).astype(np.float32)
+        with smokesim.Simulation(*dims, density=x) as g:
+            for _ in range(6):
+                same_bits(g.get_density(0), x, f"{dims}")
+    assert _pinned_calls() == 0
 
 
 def _sweep_launches(g, dt):
@@ -393,7 +411,7 @@ def case_foreign_capture():
     g.close()
 
 
-CASES = {"foreign_capture": case_foreign_capture, "read_targets": case_read_targets, "step_graph": case_step_graph, "proxy": case_proxy, "refine_groups": case_refine_groups, "single": case_single, "norms": case_norms, "plans": case_plans, "batch": case_batch,
+CASES = {"small_reads": case_small_reads, "foreign_capture": case_foreign_capture, "read_targets": case_read_targets, "step_graph": case_step_graph, "proxy": case_proxy, "refine_groups": case_refine_groups, "single": case_single, "norms": case_norms, "plans": case_plans, "batch": case_batch,
          "server": case_server, "readback": case_readback, "precision": case_precision,
          "vorticity": case_vorticity, "advection": case_advection}
 

@@ -82,6 +82,7 @@ namespace {
 
 std::map<void*, size_t> g_device, g_pinned;  // base and size
 std::map<void*, long long> g_copies;         // by device allocation: copies into it
+long long g_pinned_calls = 0;
 std::recursive_mutex g_mu;                   // held by the calls several threads make
 using Lock = std::lock_guard<std::recursive_mutex>;
 const bool g_deferred = getenv("EMU_DEFERRED") != nullptr;
@@ -355,6 +356,7 @@ hipError_t hipHostMalloc(void** p, size_t n, unsigned)
     if (unsafe_call()) return hipErrorStreamCaptureUnsupported;
     *p = malloc(n ? n : 1);
     g_pinned[*p] = n;
+    g_pinned_calls += 1;
     return hipSuccess;
 }
 hipError_t hipHostFree(void* p)
@@ -552,8 +554,9 @@ hipError_t hipEventElapsedTime(float* ms, hipEvent_t a, hipEvent_t b)
     return hipSuccess;
 }
 
-// What a test asks of the emulator: the asynchronous copies into the device
-// allocation at `base` so far.
+// What a test asks of the emulator: pinned allocations made so far, and the
+// asynchronous copies into the device allocation at `base`.
+long long emu_pinned_calls() { return g_pinned_calls; }
 long long emu_copies_into(void* base)
 {
     Lock lk(g_mu);

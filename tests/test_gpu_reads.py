@@ -9,8 +9,9 @@ import smokesim
 
 pytestmark = pytest.mark.gpu
 
-# 54 KB, 3.6 MB, 19 MB: odd sizes of the routes
-DIMS = [(29, 23, 21), (112, 100, 84), (187, 165, 160)]
+# 56 KB and just below 4 MB; just above, where pinned slots of 2 MB begin (four
+# threads), all eight threads with pieces of under 2 MB, and several each
+DIMS = [(29, 23, 21), (128, 128, 63), (128, 128, 65), (160, 151, 149), (187, 165, 160)]
 
 
 class Memory:
