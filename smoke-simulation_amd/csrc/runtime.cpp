@@ -713,21 +713,32 @@ smoke_status step_locked(smoke_sim* s, float dt)
     return SMOKE_OK;
 }
 
-// Pinned bounce buffers of the blocking reads, shared by all simulations:
-// allocated by the first read, released with the last simulation.  A reader
-// that finds them in use copies the plain way.
-constexpr int kBounceSlots = 8;
-constexpr size_t kBounceBytes = 2u << 20;
-struct Bounce {
+// Pinned slots of the blocking reads, one set per device for all of its
+// simulations, given back with the last of them.  A reader that finds them in
+// use copies the plain way.
+//
+// Page-locking them takes about 1.2 ms, so they are built only when the reads
+// that could have used them add up to their size (16 MB): a program that
+// creates a simulation, reads one field and destroys it would pay that each
+// time (create, step, read and destroy, plain / slots: 3.8 MB 0.83 / 2.1 ms,
+// 8 MB 1.8 / 3.0, 16 MB 3.0 / 2.5, 24 MB 4.4 / 3.2, 60 MB 10.6 / 7.0).
+constexpr int kReadSlots = 8, kMaxDevices = 64;
+constexpr size_t kReadSlotBytes = 2u << 20;
+struct ReadSlots {
     std::mutex mu;  // held by the reader using the slots
     char* mem = nullptr;
-    hipEvent_t ev[kBounceSlots] = {};
-    int device = -1;  // of the events
+    hipEvent_t ev[kReadSlots] = {};
+    size_t unserved = 0;       // bytes read without slots since they were given back
+    std::atomic<int> sims{0};  // live simulations of the device
 };
-Bounce g_bounce;
-std::atomic<int> g_sims{0};
+ReadSlots g_read_slots[kMaxDevices];
 
-void bounce_release(Bounce& b)
+ReadSlots* read_slots(int device)
+{
+    return device >= 0 && device < kMaxDevices ? &g_read_slots[device] : nullptr;
+}
+
+void give_back(ReadSlots& b)
 {
     for (hipEvent_t& e : b.ev) {
         if (e) (void)hipEventDestroy(e);
@@ -735,24 +746,24 @@ void bounce_release(Bounce& b)
     }
     if (b.mem) (void)hipHostFree(b.mem);
     b.mem = nullptr;
-    b.device = -1;
+    b.unserved = 0;
 }
 
-bool bounce_ready(Bounce& b, int device)
+// Whether a read of `bytes` may use the slots, on the current device.
+bool slots_ready(ReadSlots& b, size_t bytes)
 {
-    if (b.device == device) return true;
-    bounce_release(b);
-    bool ok = hipHostMalloc((void**)&b.mem, kBounceSlots * kBounceBytes, hipHostMallocDefault) == hipSuccess;
+    if (b.mem) return true;
+    b.unserved += bytes;
+    if (b.unserved < kReadSlots * kReadSlotBytes) return false;
+    bool ok = hipHostMalloc((void**)&b.mem, kReadSlots * kReadSlotBytes, hipHostMallocDefault) == hipSuccess;
     if (!ok) b.mem = nullptr;
     for (hipEvent_t& e : b.ev)
         if (ok) ok = hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
     if (!ok) {
         smk::forget_last_error();
-        bounce_release(b);
-        return false;
+        give_back(b);
     }
-    b.device = device;
-    return true;
+    return ok;
 }
 
 // Plain host memory, unknown to the GPU runtime.  Any other target (pinned,
@@ -782,27 +793,30 @@ bool pageable(const void* p)
 constexpr size_t kSlotReadBytes = 4u << 20;
 smoke_status copy_to_host(smoke_sim* s, void* dst, const void* dev, size_t bytes)
 {
-    std::unique_lock<std::mutex> lk(g_bounce.mu, std::defer_lock);
+    ReadSlots* const slots = read_slots(s->device);
+    std::unique_lock<std::mutex> lk;
+    if (slots) lk = std::unique_lock<std::mutex>(slots->mu, std::defer_lock);
     int device = -1;
     if (bytes < kSlotReadBytes || !pageable(dst) || hipGetDevice(&device) != hipSuccess ||
-        device != s->device || !lk.try_lock() || !bounce_ready(g_bounce, device)) {
+        device != s->device || !slots || !lk.try_lock() || !slots_ready(*slots, bytes)) {
+        if (lk.owns_lock()) lk.unlock();
         HIP_TRY(hipMemcpyAsync(dst, dev, bytes, hipMemcpyDeviceToHost, s->stream));
         HIP_TRY(hipStreamSynchronize(s->stream));
         return SMOKE_OK;
     }
     char* const out = static_cast<char*>(dst);
     const char* const in = static_cast<const char*>(dev);
-    const int threads = (int)std::min<size_t>(kBounceSlots, bytes >> 20);
-    const size_t width = std::min(kBounceBytes, (bytes / threads + 4095) / 4096 * 4096);
+    const int threads = (int)std::min<size_t>(kReadSlots, bytes >> 20);
+    const size_t width = std::min(kReadSlotBytes, (bytes / threads + 4095) / 4096 * 4096);
     std::atomic<int> failed{(int)hipSuccess};
     auto run = [&](int slot, bool helper) {
         hipError_t e = helper ? hipSetDevice(device) : hipSuccess;
-        char* const b = g_bounce.mem + slot * kBounceBytes;
+        char* const b = slots->mem + slot * kReadSlotBytes;
         for (size_t at = slot * width; e == hipSuccess && at < bytes; at += threads * width) {
             const size_t n = std::min(width, bytes - at);
             e = hipMemcpyAsync(b, in + at, n, hipMemcpyDeviceToHost, s->stream);
-            if (e == hipSuccess) e = hipEventRecord(g_bounce.ev[slot], s->stream);
-            if (e == hipSuccess) e = hipEventSynchronize(g_bounce.ev[slot]);
+            if (e == hipSuccess) e = hipEventRecord(slots->ev[slot], s->stream);
+            if (e == hipSuccess) e = hipEventSynchronize(slots->ev[slot]);
             if (e == hipSuccess) std::memcpy(out + at, b, n);
         }
         if (e != hipSuccess) failed = (int)e;
@@ -910,7 +924,6 @@ smoke_status smoke_create_ex(unsigned nx, unsigned ny, unsigned nz, const float*
                     nx, ny, nz);
     if (!storage_ok(storage)) return fail(SMOKE_ERR_INVALID, "create: unknown storage %d", storage);
     smoke_sim* s = new smoke_sim();
-    ++g_sims;
     s->g = make_grid(nx, ny, nz);
     s->storage = storage;
     smoke_params_default(&s->prm);
@@ -921,7 +934,11 @@ smoke_status smoke_create_ex(unsigned nx, unsigned ny, unsigned nz, const float*
         return st;
     };
     hipError_t e = hipGetDevice(&s->device);
-    if (e != hipSuccess) return bail(fail(SMOKE_ERR_HIP, "create: no device: %s", hipGetErrorString(e)));
+    if (e != hipSuccess) {
+        s->device = -1;
+        return bail(fail(SMOKE_ERR_HIP, "create: no device: %s", hipGetErrorString(e)));
+    }
+    if (ReadSlots* b = read_slots(s->device)) ++b->sims;
     e = hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking);
     if (e != hipSuccess) return bail(fail(SMOKE_ERR_HIP, "create: stream: %s", hipGetErrorString(e)));
     size_t bytes = arena_bytes(s->g, storage);
@@ -1009,10 +1026,11 @@ void smoke_destroy(smoke_sim* s)
     if (s->norms_mem) (void)hipFree(s->norms_mem);
     if (s->arena) (void)hipFree(s->arena);
     if (s->stream) (void)hipStreamDestroy(s->stream);
+    ReadSlots* const slots = read_slots(s->device);
     delete s;
-    if (--g_sims == 0) {
-        std::lock_guard<std::mutex> lk(g_bounce.mu);
-        if (g_sims == 0) bounce_release(g_bounce);
+    if (slots && --slots->sims == 0) {
+        std::lock_guard<std::mutex> lk(slots->mu);
+        if (slots->sims == 0) give_back(*slots);
     }
 }
 

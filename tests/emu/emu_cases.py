@@ -362,11 +362,11 @@ def case_read_targets():
         g.close()
 
 
-def _pinned_calls():
+def _emu(name, *args):
     import ctypes
-    f = smokesim.load().emu_pinned_calls
+    f = getattr(smokesim.load(), name)
     f.restype = ctypes.c_longlong
-    return f()
+    return f(*[ctypes.c_size_t(a) for a in args])
 
 
 def case_small_reads():
@@ -377,7 +377,47 @@ def case_small_reads():
         with smokesim.Simulation(*dims, density=x) as g:
             for _ in range(6):
                 same_bits(g.get_density(0), x, f"{dims}")
-    assert _pinned_calls() == 0
+    assert _emu("emu_pinned_calls") == 0
+
+
+def case_read_slots():
+    # The pinned slots of the blocking reads: built once the reads add up to
+    # their size, one set per device, kept while a simulation of the device
+    # lives, and refused without harm.
+    lib = smokesim.load()
+    dims = (120, 100, 91)  # 4.2 MB
+    x = np.random.default_rng(13).standard_normal(dims[::-1]).astype(np.float32)
+
+    def read(g, n, what):
+        for _ in range(n):
+            same_bits(g.get_density(0), x, what)
+
+    for k in range(5):  # too little is read in any one life
+        with smokesim.Simulation(*dims, density=x) as g:
+            read(g, 2, f"life {k}")
+    assert _emu("emu_pinned_calls") == 0
+    sims = []
+    for d in (0, 1):
+        assert lib.hipSetDevice(d) == 0
+        sims.append(smokesim.Simulation(*dims, density=x))
+    for k in range(8):
+        for d, g in enumerate(sims):
+            assert lib.hipSetDevice(d) == 0
+            read(g, 1, f"device {d} read {k}")
+    assert _emu("emu_pinned_calls") == 2 and _emu("emu_pinned_held") == 2
+    sims[0].close()
+    assert _emu("emu_pinned_held") == 1
+    sims[1].close()
+    assert _emu("emu_pinned_held") == 0
+    assert lib.hipSetDevice(0) == 0
+    with smokesim.Simulation(*dims, density=x) as g:
+        _emu("emu_refuse_above", 4 << 20)
+        read(g, 9, "refused")
+        assert _emu("emu_pinned_calls") == 4 and _emu("emu_pinned_held") == 0
+        _emu("emu_refuse_above", 2 ** 63)
+        read(g, 5, "later")
+        assert _emu("emu_pinned_held") == 1
+    assert _emu("emu_pinned_held") == 0
 
 
 def _sweep_launches(g, dt):
@@ -411,7 +451,7 @@ def case_foreign_capture():
     g.close()
 
 
-CASES = {"small_reads": case_small_reads, "foreign_capture": case_foreign_capture, "read_targets": case_read_targets, "step_graph": case_step_graph, "proxy": case_proxy, "refine_groups": case_refine_groups, "single": case_single, "norms": case_norms, "plans": case_plans, "batch": case_batch,
+CASES = {"read_slots": case_read_slots, "small_reads": case_small_reads, "foreign_capture": case_foreign_capture, "read_targets": case_read_targets, "step_graph": case_step_graph, "proxy": case_proxy, "refine_groups": case_refine_groups, "single": case_single, "norms": case_norms, "plans": case_plans, "batch": case_batch,
          "server": case_server, "readback": case_readback, "precision": case_precision,
          "vorticity": case_vorticity, "advection": case_advection}
 

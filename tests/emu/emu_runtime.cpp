@@ -83,6 +83,7 @@ namespace {
 std::map<void*, size_t> g_device, g_pinned;  // base and size
 std::map<void*, long long> g_copies;         // by device allocation: copies into it
 long long g_pinned_calls = 0;
+size_t g_refuse_above = SIZE_MAX;  // larger allocations are refused
 std::recursive_mutex g_mu;                   // held by the calls several threads make
 using Lock = std::lock_guard<std::recursive_mutex>;
 const bool g_deferred = getenv("EMU_DEFERRED") != nullptr;
@@ -105,6 +106,7 @@ void check(hipStream_t s)
 {
     if (s && s->magic != kStream) die("use of an invalid stream");
 }
+thread_local int t_device = 0;  // of two devices
 // A call that captures forbid: true, and the captures are ended, unless this
 // thread's mode allows it.
 thread_local hipStreamCaptureMode t_mode = hipStreamCaptureModeGlobal;
@@ -354,9 +356,10 @@ hipError_t hipHostMalloc(void** p, size_t n, unsigned)
 {
     Lock lk(g_mu);
     if (unsafe_call()) return hipErrorStreamCaptureUnsupported;
+    g_pinned_calls += 1;
+    if (n > g_refuse_above) return hipErrorOutOfMemory;
     *p = malloc(n ? n : 1);
     g_pinned[*p] = n;
-    g_pinned_calls += 1;
     return hipSuccess;
 }
 hipError_t hipHostFree(void* p)
@@ -392,10 +395,15 @@ hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipSt
 }
 hipError_t hipGetDevice(int* d)
 {
-    *d = 0;
+    *d = t_device;
     return hipSuccess;
 }
-hipError_t hipSetDevice(int d) { return d == 0 ? hipSuccess : hipErrorInvalidDevice; }
+hipError_t hipSetDevice(int d)
+{
+    if (d < 0 || d > 1) return hipErrorInvalidDevice;
+    t_device = d;
+    return hipSuccess;
+}
 hipError_t hipGetSymbolAddress(void** p, const void* symbol)
 {
     *p = const_cast<void*>(symbol);
@@ -554,9 +562,12 @@ hipError_t hipEventElapsedTime(float* ms, hipEvent_t a, hipEvent_t b)
     return hipSuccess;
 }
 
-// What a test asks of the emulator: pinned allocations made so far, and the
-// asynchronous copies into the device allocation at `base`.
+// What a test asks of the emulator: pinned allocations asked for so far and
+// held now, the asynchronous copies into the device allocation at `base`; and
+// to refuse allocations of more than n bytes.
 long long emu_pinned_calls() { return g_pinned_calls; }
+long long emu_pinned_held() { return (long long)g_pinned.size(); }
+void emu_refuse_above(size_t n) { g_refuse_above = n; }
 long long emu_copies_into(void* base)
 {
     Lock lk(g_mu);

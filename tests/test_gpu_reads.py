@@ -1,6 +1,7 @@
 """Blocking reads of a field: the same values whatever memory the caller gives
 (plain, pinned or device memory) and whatever route the size takes."""
 import ctypes
+import threading
 
 import numpy as np
 import pytest
@@ -49,3 +50,37 @@ def test_read_targets(dims, kind):
         assert np.array_equal(m.floats(), x.ravel())
         m.free()
         assert np.array_equal(g.get_density(0), x)
+
+
+def test_readers_at_once():
+    # One reader has the slots, the others copy the plain way.
+    rng = np.random.default_rng(4)
+    sims = [(smokesim.Simulation(*d), rng.standard_normal(d[::-1]).astype(np.float32))
+            for d in [DIMS[4], DIMS[2], DIMS[4], DIMS[3]]]
+    wrong = []
+
+    def work(g, x):
+        for k in range(8):
+            y = x * np.float32(k + 1)
+            g.set_density(0, y)
+            if not np.array_equal(g.get_density(0), y):
+                wrong.append((g.cell_shape, k))
+
+    threads = [threading.Thread(target=work, args=p) for p in sims]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
+    for g, _ in sims:
+        g.close()
+
+
+def test_lives_of_one_read():
+    # Simulations that are created, read and destroyed, below and above the
+    # size at which the slots are built.
+    x = np.random.default_rng(5).standard_normal(DIMS[4][::-1]).astype(np.float32)
+    for k, n in enumerate([70, 160, 30, 160, 160]):
+        y = x[:n]
+        with smokesim.Simulation(187, 165, n, density=y) as g:
+            assert np.array_equal(g.get_density(0), y), k
