@@ -468,9 +468,7 @@ __global__ __launch_bounds__(TP * TY) void k_ref_pressure_march(
     }
 }
 
-// Planes per workgroup of the marched forms, one workgroup per CU (1024
-// threads), and the steps of the busiest CU: a workgroup's steps are its planes
-// and the pipeline's fill.
+// Launch of a marched form: columns in x and y, chunks of zc planes in z.
 struct MarchPlan {
     dim3 grid;
     int zc;
@@ -478,18 +476,8 @@ struct MarchPlan {
 };
 inline MarchPlan march_plan(int nx, int ny, int planes, int fill)
 {
-    MarchPlan p = {dim3(), planes, -1};
-    for (int chunks = 1; chunks <= (planes + 1) / 2; ++chunks) {
-        const int zc = (planes + chunks - 1) / chunks;
-        const long long rounds = ((long long)nx * ny * ((planes + zc - 1) / zc) + kCUs - 1) / kCUs;
-        const long long steps = rounds * (zc + fill);
-        if (p.steps < 0 || steps < p.steps) {
-            p.steps = steps;
-            p.zc = zc;
-        }
-    }
-    p.grid = dim3((unsigned)nx, (unsigned)ny, (unsigned)((planes + p.zc - 1) / p.zc));
-    return p;
+    const MarchChunk c = fit_march((long long)nx * ny, planes, fill);
+    return {dim3((unsigned)nx, (unsigned)ny, (unsigned)((planes + c.zc - 1) / c.zc)), c.zc, c.steps};
 }
 
 constexpr int kMarchTP = 32, kMarchTY = 32;

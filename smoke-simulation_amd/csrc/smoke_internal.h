@@ -138,6 +138,28 @@ inline int fit_chunk(const ChunkModel& m, int tiles, int planes, int most, doubl
     *us = best_us;
     return best;
 }
+// Planes per workgroup of the marched red-black forms (redblack.h), one
+// workgroup per CU: the fewest steps of the busiest CU, a workgroup's steps
+// being its planes and the pipeline's `fill`.  The search ends where even an
+// equal share of all steps per CU is no fewer than the best found: after at most
+// 290 of the counts of chunks, 1.5 us a call, where trying them all took 12 us
+// for 4000 planes and 120 for 50000, on every launch.
+struct MarchChunk {
+    int zc;
+    long long steps;
+};
+inline MarchChunk fit_march(long long columns, int planes, int fill)
+{
+    MarchChunk best{planes, -1};
+    for (int chunks = 1; chunks <= (planes + 1) / 2; ++chunks) {
+        if (best.steps >= 0 && columns * (planes + (long long)chunks * fill) >= best.steps * kCUs) break;
+        const int zc = (planes + chunks - 1) / chunks;
+        const long long rounds = (columns * ((planes + zc - 1) / zc) + kCUs - 1) / kCUs;
+        const long long steps = rounds * (zc + fill);
+        if (best.steps < 0 || steps < best.steps) best = {zc, steps};
+    }
+    return best;
+}
 // The plan of a simulation whose plan was never set (step_kernels.hip), for
 // the Jacobi sweeps and for the refined solve's FP16 sweeps.
 JacobiPlan fitted_plan(const Grid& g, bool refined);
