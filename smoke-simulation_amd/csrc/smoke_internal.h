@@ -140,23 +140,27 @@ inline int fit_chunk(const ChunkModel& m, int tiles, int planes, int most, doubl
 }
 // Planes per workgroup of the marched red-black forms (redblack.h), one
 // workgroup per CU: the fewest steps of the busiest CU, a workgroup's steps
-// being its planes and the pipeline's `fill`.  The search ends where even an
-// equal share of all steps per CU is no fewer than the best found: after at most
-// 290 of the counts of chunks, 1.5 us a call, where trying them all took 12 us
-// for 4000 planes and 120 for 50000, on every launch.
+// being its planes and the pipeline's `fill`.  For each number of rounds over the
+// CUs only the most chunks that fit it count, and the search ends where the
+// grid's planes and the fill of that many rounds are no fewer steps than the best
+// found: a few counts instead of all of them, which took 12 us for 4000 planes
+// and 120 for 50000, on every launch.
 struct MarchChunk {
     int zc;
     long long steps;
 };
 inline MarchChunk fit_march(long long columns, int planes, int fill)
 {
+    const long long most = (planes + 1) / 2;
     MarchChunk best{planes, -1};
-    for (int chunks = 1; chunks <= (planes + 1) / 2; ++chunks) {
-        if (best.steps >= 0 && columns * (planes + (long long)chunks * fill) >= best.steps * kCUs) break;
-        const int zc = (planes + chunks - 1) / chunks;
-        const long long rounds = (columns * ((planes + zc - 1) / zc) + kCUs - 1) / kCUs;
-        const long long steps = rounds * (zc + fill);
+    for (long long rounds = (columns + kCUs - 1) / kCUs;; ++rounds) {
+        if (best.steps >= 0 && columns * planes + rounds * fill * kCUs >= best.steps * kCUs) break;
+        const long long fit = rounds * kCUs / columns, chunks = fit < most ? fit : most;
+        const int zc = (int)((planes + chunks - 1) / chunks);
+        const long long used = (columns * ((planes + zc - 1) / zc) + kCUs - 1) / kCUs;
+        const long long steps = used * (zc + fill);
         if (best.steps < 0 || steps < best.steps) best = {zc, steps};
+        if (chunks == most) break;
     }
     return best;
 }
