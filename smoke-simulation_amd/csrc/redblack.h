@@ -496,13 +496,11 @@ struct FaceSets {
 };
 
 template <int H>
-hipError_t launch_faces_march(const Grid& g, const FaceSets& f, const uint8_t* flags, int colour,
-                              int sweeps, double omega, hipStream_t st)
+hipError_t launch_faces_march(const Grid& g, const MarchPlan& p, const FaceSets& f, const uint8_t* flags,
+                              int colour, int sweeps, double omega, hipStream_t st)
 {
-    const MarchPlan p = faces_plan<H>(g);
-    const int zc = p.zc;
     hipLaunchKernelGGL((k_ref_faces_march<kMarchTP, kMarchTY, H>), p.grid, dim3(kMarchTP, kMarchTY), 0,
-                       st, g, f.ui, f.vi, f.wi, f.uo, f.vo, f.wo, flags, zc, colour, sweeps, omega);
+                       st, g, f.ui, f.vi, f.wi, f.uo, f.vo, f.wo, flags, p.zc, colour, sweeps, omega);
     return hipGetLastError();
 }
 

@@ -260,11 +260,13 @@ struct AllowWhileCapturing {
 };
 
 // Allocates the reference projection's second velocity set (once per
-// simulation, before a step or a capture of its own).  Its launches write
-// every entry they later read.
+// simulation, before a step or a capture of its own, where its launches are
+// the faster ones).  They write every entry they later read.
 void ensure_sweep_fields(smoke_sim* s)
 {
-    if (s->prm.projection != SMOKE_PROJ_REFERENCE || s->sweep_mem || s->sweep_refused) return;
+    if (s->prm.projection != SMOKE_PROJ_REFERENCE || s->sweep_mem || s->sweep_refused ||
+        smk::reference_in_place(s->g, 2 * s->prm.iterations))
+        return;
     const AllowWhileCapturing allow;
     const size_t field = align256((size_t)s->g.elems * sizeof(float));
     if (hipMalloc((void**)&s->sweep_mem, 3 * field) != hipSuccess) {
@@ -459,7 +461,7 @@ hipError_t stage_project(smoke_sim* s, long long* launches)
         }
         if ((e = sweep_mark(s, 0, 0)) != hipSuccess) return e;
         int n_launches = 2 * p.iterations;
-        if (s->sweep_mem && p.iterations >= 2) {
+        if (s->sweep_mem && !smk::reference_in_place(g, n_launches)) {
             float* const vel[3] = {s->u[n], s->v[n], s->w[n]};
             e = smk::project_reference_sweeps(g, vel, s->sweep_vel, s->flags, 2 * p.iterations,
                                               p.sor_omega, s->stream, &n_launches);

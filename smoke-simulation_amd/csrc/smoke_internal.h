@@ -318,6 +318,9 @@ void forget_last_error();
 // Projection.
 hipError_t project_reference_half(const Grid& g, float* u, float* v, float* w,
                                   const uint8_t* flags, int colour, double omega, hipStream_t st);
+// Whether `sweeps` half-sweeps are faster as that many launches in place than by
+// project_reference_sweeps.
+bool reference_in_place(const Grid& g, int sweeps);
 // `sweeps` half-sweeps (an even number, at least 2) in a few launches
 // (redblack.h), alternating between the fields a (u, v, w) and b (three
 // scratch fields of the same layout); the result is in a.

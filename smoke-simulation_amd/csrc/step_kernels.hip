@@ -662,27 +662,66 @@ hipError_t project_reference_half(const Grid& g, float* u, float* v, float* w,
     return hipGetLastError();
 }
 
+// How the reference form's half-sweeps run.  At most one box per CU: boxes
+// (redblack.h has both sides).  Else columns, 4 half-sweeps per launch, or where
+// the two sets of faces and the flags approach the 256 MB memory-side cache (a
+// launch is then bound by memory and fewer passes pay for the larger halo) the
+// better fitting of 5 and 6.  us per half-sweep with 4 / 5 / 6: 160^3 (125 MB)
+// 8.6 / 10.0 / 9.5, 192x180x188 (191 MB) 11.6 / 11.9 / 11.7, 224x200x210 (271 MB)
+// 19.7 / 16.9 / 16.0, 256x240x248 29.4 / 26.6 / 29.0 (one column more for 6).
+constexpr int kBoxX = 24, kBoxY = 10, kBoxZ = 10;
+struct FacesRoute {
+    bool boxed;
+    dim3 boxes;
+    int H;
+    MarchPlan plan;  // of the columns
+};
+static FacesRoute faces_route(const Grid& g)
+{
+    FacesRoute r{};
+    r.boxes = dim3((unsigned)((g.nx + kBoxX - 1) / kBoxX), (unsigned)((g.ny + kBoxY - 1) / kBoxY),
+                   (unsigned)((g.nz + kBoxZ - 1) / kBoxZ));
+    r.boxed = (long long)r.boxes.x * r.boxes.y * r.boxes.z <= kCUs;
+    r.H = 4;
+    if (r.boxed) return r;
+    if ((long long)g.elems * 25 > (180LL << 20)) {
+        const MarchPlan five = faces_plan<5>(g), six = faces_plan<6>(g);
+        r.H = five.steps * 6 < six.steps * 5 ? 5 : 6;
+        r.plan = r.H == 5 ? five : six;
+    } else {
+        r.plan = faces_plan<4>(g);
+    }
+    return r;
+}
+// An even number of launches, so that the last one writes the first set again.
+static int faces_launches(const FacesRoute& r, int sweeps) { return 2 * ((sweeps + 2 * r.H - 1) / (2 * r.H)); }
+
+// A column of the marched launches costs the same however few of its cells the
+// grid has, and a grid thin in x or y fills little of it: one half-sweep per
+// launch in place is then faster.  Both by their measured times (400 random
+// grids, extents 3..20000, within 5 % for most): a marched launch 2.5 us and 1.1
+// a step, a half-sweep 2.8 us, 6.9 per 10^5 128-byte lines and 3.4 per 10^6
+// cells.  The march has to gain 15 % by these.  us for 40 half-sweeps, in place /
+// marched: 18072x3x56 290 / 1290, 59x4x19372 569 / 1864, 10x4x3220 146 / 299,
+// 129x9x882 249 / 282, 130x3308x6 388 / 412; 28x120x289 326 / 226, 150x96x121
+// 431 / 226.
+bool reference_in_place(const Grid& g, int sweeps)
+{
+    if (sweeps < 4) return true;
+    if ((g.nz - 2 + kRefZ - 1) / kRefZ > 65535) return false;  // a grid's y extent
+    const FacesRoute r = faces_route(g);
+    if (r.boxed) return false;
+    const double rows = (double)(g.ny - 2) * (g.nz - 2), lines = rows * ((g.nx + 31) / 32);
+    const double in_place = sweeps * (2.8 + 6.9e-5 * lines + 3.4e-6 * rows * (g.nx - 2));
+    return in_place < 1.15 * faces_launches(r, sweeps) * (2.5 + 1.1 * (double)r.plan.steps);
+}
+
 hipError_t project_reference_sweeps(const Grid& g, float* const (&a)[3], float* const (&b)[3],
                                     const uint8_t* flags, int sweeps, double omega, hipStream_t st,
                                     int* launches)
 {
-    // At most one box per CU: boxes (redblack.h has both sides).  Else columns,
-    // 4 half-sweeps per launch, or where the two sets of faces and the flags
-    // approach the 256 MB memory-side cache (a launch is then bound by memory
-    // and fewer passes pay for the larger halo) the better fitting of 5 and 6.
-    // us per half-sweep with 4 / 5 / 6: 160^3 (125 MB) 8.6 / 10.0 / 9.5,
-    // 192x180x188 (191 MB) 11.6 / 11.9 / 11.7, 224x200x210 (271 MB) 19.7 /
-    // 16.9 / 16.0, 256x240x248 29.4 / 26.6 / 29.0 (one column more for 6).
-    constexpr int IX = 24, IY = 10, IZ = 10;
-    const dim3 boxes((unsigned)((g.nx + IX - 1) / IX), (unsigned)((g.ny + IY - 1) / IY),
-                     (unsigned)((g.nz + IZ - 1) / IZ));
-    const bool boxed = (long long)boxes.x * boxes.y * boxes.z <= kCUs;
-    const bool large = (long long)g.elems * 25 > (180LL << 20);
-    int H = 4;
-    if (!boxed && large)
-        H = faces_plan<5>(g).steps * 6 < faces_plan<6>(g).steps * 5 ? 5 : 6;
-    // An even number of launches, so that the last one writes a again.
-    const int n = 2 * ((sweeps + 2 * H - 1) / (2 * H));
+    const FacesRoute r = faces_route(g);
+    const int n = faces_launches(r, sweeps);
     *launches = 0;
     for (int l = 0, done = 0; l < n; ++l) {
         const int m = sweeps / n + (l < sweeps % n ? 1 : 0), colour = done & 1;
@@ -690,14 +729,14 @@ hipError_t project_reference_sweeps(const Grid& g, float* const (&a)[3], float* 
         float* const* out = l & 1 ? a : b;
         const FaceSets f = {in[0], in[1], in[2], out[0], out[1], out[2]};
         hipError_t e;
-        if (boxed) {
-            hipLaunchKernelGGL((k_ref_faces_box<IX, IY, IZ, 4>), boxes, dim3(kBoxThreads), 0, st, g,
-                               f.ui, f.vi, f.wi, f.uo, f.vo, f.wo, flags, colour, m, omega);
+        if (r.boxed) {
+            hipLaunchKernelGGL((k_ref_faces_box<kBoxX, kBoxY, kBoxZ, 4>), r.boxes, dim3(kBoxThreads), 0,
+                               st, g, f.ui, f.vi, f.wi, f.uo, f.vo, f.wo, flags, colour, m, omega);
             e = hipGetLastError();
         } else {
-            e = H == 6   ? launch_faces_march<6>(g, f, flags, colour, m, omega, st)
-                : H == 5 ? launch_faces_march<5>(g, f, flags, colour, m, omega, st)
-                         : launch_faces_march<4>(g, f, flags, colour, m, omega, st);
+            e = r.H == 6   ? launch_faces_march<6>(g, r.plan, f, flags, colour, m, omega, st)
+                : r.H == 5 ? launch_faces_march<5>(g, r.plan, f, flags, colour, m, omega, st)
+                           : launch_faces_march<4>(g, r.plan, f, flags, colour, m, omega, st);
         }
         if (e != hipSuccess) return e;
         done += m;

@@ -430,6 +430,22 @@ def _sweep_launches(g, dt):
     return n
 
 
+def case_thin_reference():
+    # Grids whose columns would be mostly empty run one half-sweep per launch,
+    # others several, with the same bits; a change of the iteration count may
+    # change the route.
+    for dims, its, several in [((3, 4, 2700), 3, False), ((3, 2700, 4), 3, False),
+                               ((14, 12, 10), 3, True), ((14, 12, 10), 1, False)]:
+        sc = scenes.test_scene(dims, seed=38, projection=0, iterations=its, box_fraction=0.0,
+                               n_obstacles=0)
+        g, o = gpu_for(sc), oracle_for(sc, 32)
+        n = _sweep_launches(g, sc["dt"])
+        assert (n < 2 * its) == several, (dims, its, n)
+        o.step(sc["dt"], 1)
+        assert_bitwise_equal(g.state(), o.state(), f"thin {dims} x{its}")
+        g.close()
+
+
 def case_foreign_capture():
     # A first step of the reference form while another stream is captured in
     # the global mode: the capture goes on, and this and later steps run
@@ -451,7 +467,7 @@ def case_foreign_capture():
     g.close()
 
 
-CASES = {"read_slots": case_read_slots, "small_reads": case_small_reads, "foreign_capture": case_foreign_capture, "read_targets": case_read_targets, "step_graph": case_step_graph, "proxy": case_proxy, "refine_groups": case_refine_groups, "single": case_single, "norms": case_norms, "plans": case_plans, "batch": case_batch,
+CASES = {"thin_reference": case_thin_reference, "read_slots": case_read_slots, "small_reads": case_small_reads, "foreign_capture": case_foreign_capture, "read_targets": case_read_targets, "step_graph": case_step_graph, "proxy": case_proxy, "refine_groups": case_refine_groups, "single": case_single, "norms": case_norms, "plans": case_plans, "batch": case_batch,
          "server": case_server, "readback": case_readback, "precision": case_precision,
          "vorticity": case_vorticity, "advection": case_advection}
 
