@@ -350,8 +350,8 @@ __global__ __launch_bounds__(TP * TY) void k_ref_faces_march(
 //
 // us per half-sweep, one per launch before: 113x90x101 6.3 -> 3.2, 80^3 4.5 ->
 // 2.6, 256x240x248 44 -> 11.8.  Small grids are a chain of LDS latencies and
-// barriers (16-pair columns, two per CU, then beat 32-pair ones: 48x40x57 2.1
-// against 2.7), large ones 3.5 TB/s of loads and stores over VALU issue.
+// barriers (16-pair columns of half the threads then beat 32-pair ones: 48x40x57
+// 2.1 against 2.7), large ones 3.5 TB/s of loads and stores over VALU issue.
 template <int TP, int TY, int H>
 struct PressureColumn {
     static_assert(H % 2 == 0 && 64 % TP == 0, "whole pairs, whole rows per wave");
@@ -512,14 +512,12 @@ MarchPlan pressure_plan(const Grid& g)
 }
 
 template <int TP, int H>
-hipError_t launch_pressure_march(const Grid& g, const float* pi, float* po, const float* d,
-                                 const uint8_t* flags, int colour, int sweeps, float omega, int cold,
-                                 hipStream_t st)
+hipError_t launch_pressure_march(const Grid& g, const MarchPlan& p, const float* pi, float* po,
+                                 const float* d, const uint8_t* flags, int colour, int sweeps,
+                                 float omega, int cold, hipStream_t st)
 {
-    const MarchPlan p = pressure_plan<TP, H>(g);
-    const int zc = p.zc;
     hipLaunchKernelGGL((k_ref_pressure_march<TP, kMarchTY, H>), p.grid, dim3(TP, kMarchTY), 0, st, g, pi,
-                       po, d, flags, zc, colour, sweeps, omega, cold);
+                       po, d, flags, p.zc, colour, sweeps, omega, cold);
     return hipGetLastError();
 }
 

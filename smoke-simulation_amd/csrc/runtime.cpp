@@ -506,18 +506,26 @@ hipError_t stage_project(smoke_sim* s, long long* launches)
         *launches += sweep_launches;
         if ((e = sweep_mark(s, 1, sweep_launches)) != hipSuccess) return e;
     } else {
-        int n_launches = 0;
-        if (p.iterations == 0) {
-            // No half-sweeps: P = 0, or the last step's on the active cells.
+        int n_launches = 2 * p.iterations;
+        const bool in_place = smk::rbsor_in_place(g, n_launches);
+        if (in_place) {
+            // From P = 0, or from the last step's on the active cells.
             e = p.warm_start ? smk::mask_pressure(g, s->P[s->pcur], s->flags, s->stream)
                              : smk::fill_f32(s->P[s->pcur], g.elems, 0.0f, s->stream);
             if (e != hipSuccess) return e;
             *launches += 1;
         }
         if ((e = sweep_mark(s, 0, 0)) != hipSuccess) return e;
-        e = smk::rbsor_sweeps(g, s->P, &s->pcur, s->d, s->flags, 2 * p.iterations, (float)p.sor_omega,
-                              !p.warm_start, s->stream, &n_launches);
-        if (e != hipSuccess) return e;
+        if (in_place) {
+            for (int k = 0; k < n_launches; ++k) {
+                e = smk::rbsor_half(g, s->P[s->pcur], s->d, s->flags, k & 1, (float)p.sor_omega, s->stream);
+                if (e != hipSuccess) return e;
+            }
+        } else {
+            e = smk::rbsor_sweeps(g, s->P, &s->pcur, s->d, s->flags, n_launches, (float)p.sor_omega,
+                                  !p.warm_start, s->stream, &n_launches);
+            if (e != hipSuccess) return e;
+        }
         *launches += n_launches;
         if ((e = sweep_mark(s, 1, n_launches)) != hipSuccess) return e;
     }

@@ -341,6 +341,11 @@ hipError_t jacobi_fused(const Grid& g, const float* pin, float* pout, const floa
 hipError_t rbsor_sweeps(const Grid& g, float* const (&p)[2], int* cur, const float* d,
                         const uint8_t* flags, int sweeps, float omega, int cold, hipStream_t st,
                         int* launches);
+// Whether `sweeps` half-sweeps are faster as that many launches of rbsor_half, in
+// place on a pressure that is 0 on cells that are not active.
+bool rbsor_in_place(const Grid& g, int sweeps);
+hipError_t rbsor_half(const Grid& g, float* p, const float* d, const uint8_t* flags, int colour,
+                      float omega, hipStream_t st);
 hipError_t mask_pressure(const Grid& g, float* p, const uint8_t* flags, hipStream_t st);
 hipError_t gradient(const Grid& g, float* u, float* v, float* w, const float* p,
                     const uint8_t* flags, hipStream_t st);

@@ -367,6 +367,55 @@ __global__ __launch_bounds__(TX * TY / R, 8 / R) void k_jacobi_fused(
                                                  L % nbx, (L / nbx) % nby, L / (nbx * nby), sh);
 }
 
+// One red-black SOR half-sweep of the pressure form, in place (on grids thin in
+// x or y, rbsor_in_place).
+__global__ __launch_bounds__(BX * BY) void k_rbsor_half(Grid g, float* __restrict__ p,
+                                                    const float* __restrict__ d,
+                                                    const uint8_t* __restrict__ flags, int colour,
+                                                    float omega, int pairs)
+{
+    // The same thread layout as k_project_ref_half: a flat (column pair, row)
+    // index and kRefZ consecutive planes per thread, every load issued before
+    // any update.  The neighbours are of the other colour, which this launch
+    // leaves alone, and every interior cell's neighbours lie inside the array.
+    const int f = (int)blockIdx.x * (BX * BY) + (int)threadIdx.y * BX + (int)threadIdx.x;
+    if (f >= pairs * (g.ny - 2)) return;
+    const int t = f % pairs, y = f / pairs + 1;
+    const int z0 = (int)blockIdx.y * kRefZ + 1;
+    float nb[kRefZ][6], pc[kRefZ], di[kRefZ];
+    uint8_t fl[kRefZ];
+    int ic[kRefZ];
+#pragma unroll
+    for (int j = 0; j < kRefZ; ++j) {
+        const int z = z0 + j, x = dev::colour_x(t, y, z, colour);
+        fl[j] = 0;
+        ic[j] = 0;
+        pc[j] = di[j] = 0.0f;
+#pragma unroll
+        for (int k = 0; k < 6; ++k) nb[j][k] = 0.0f;
+        if (z > g.nz - 2 || x > g.nx - 2) continue;
+        const int i = g.idx(x, y, z);
+        ic[j] = i;
+        nb[j][0] = p[i - 1];
+        nb[j][1] = p[i + 1];
+        nb[j][2] = p[i - g.px];
+        nb[j][3] = p[i + g.px];
+        nb[j][4] = p[i - g.plane];
+        nb[j][5] = p[i + g.plane];
+        pc[j] = p[i];
+        di[j] = d[i];
+        fl[j] = flags[i];
+    }
+#pragma unroll
+    for (int j = 0; j < kRefZ; ++j) {
+        if (!(fl[j] & F_ACTIVE)) continue;
+        const float G = dev::pressure_update(
+            dev::sum6(nb[j][0], nb[j][1], nb[j][2], nb[j][3], nb[j][4], nb[j][5]),
+            dev::inv_acc(__popc(fl[j] & F_NBRS)), di[j]);
+        p[ic[j]] = pc[j] + omega * (G - pc[j]);
+    }
+}
+
 // Warm start: zero the pressure of cells that are not active.
 __global__ void k_mask_pressure(Grid g, float* __restrict__ p, const uint8_t* __restrict__ flags)
 {
@@ -865,18 +914,66 @@ hipError_t jacobi_fused(const Grid& g, const float* pin, float* pout, const floa
     }
 }
 
+// 4 or 6 half-sweeps per launch, whichever takes fewer steps per half-sweep;
+// narrow columns where the grid is too small to fill the CUs with wide ones.
+// us per half-sweep, narrow 4 / 4 / 6: 48x40x57 2.1 / 2.8 / 2.7, 80^3 2.6 / 2.9
+// / 2.8, 113x90x101 3.2 / 3.3 / 3.4, 150^3 4.8 / 5.0 / 4.7, 256x240x248 13.3 /
+// 12.3 / 11.8.
+struct PressureRoute {
+    bool narrow;
+    int H;
+    MarchPlan plan;
+};
+static PressureRoute pressure_route(const Grid& g)
+{
+    PressureRoute r{(long long)g.nx * g.ny * g.nz <= 1500000, 4, MarchPlan{}};
+    if (r.narrow) {
+        r.plan = pressure_plan<16, 4>(g);
+        return r;
+    }
+    const MarchPlan four = pressure_plan<32, 4>(g), six = pressure_plan<32, 6>(g);
+    r.H = four.steps * 6 <= six.steps * 4 ? 4 : 6;
+    r.plan = r.H == 4 ? four : six;
+    return r;
+}
+
+// As reference_in_place, by the pressure form's times (1200 random grids): a
+// marched launch 2.5 us and 0.86 a step of wide columns, 0.535 of narrow ones
+// (0.39 where two of those share a CU); a half-sweep 2.35 us, 4.2 per 10^5
+// 128-byte lines and 2.3 per 10^6 cells, and one pass to mask or clear the
+// pressure.  The march has to gain 10 %.  us for 40 half-sweeps with divergence
+// and gradient, in place / marched: 18072x3x56 249 / 728, 51x4x6934 221 / 522,
+// 3944x209x3 207 / 270, 256x6x235 139 / 143; 24^3 122 / 93, 113x90x101 265 / 147.
+bool rbsor_in_place(const Grid& g, int sweeps)
+{
+    if (sweeps == 0) return true;
+    if ((g.nz - 2 + kRefZ - 1) / kRefZ > 65535) return false;  // a grid's y extent
+    const PressureRoute r = pressure_route(g);
+    const double rows = (double)(g.ny - 2) * (g.nz - 2), lines = rows * ((g.nx + 31) / 32);
+    const double in_place = sweeps * (2.35 + 4.2e-5 * lines + 2.3e-6 * rows * (g.nx - 2)) + 2.3 + 1e-6 * g.elems;
+    const bool shared = (long long)r.plan.grid.x * r.plan.grid.y * r.plan.grid.z > kCUs;
+    const double step = r.narrow ? (shared ? 0.39 : 0.535) : 0.86;
+    return in_place < 1.1 * sweeps / r.H * (2.5 + step * (double)r.plan.steps);
+}
+
+hipError_t rbsor_half(const Grid& g, float* p, const float* d, const uint8_t* flags, int colour,
+                      float omega, hipStream_t st)
+{
+    const int pairs = (g.nx - 2 + 1) / 2;
+    const long long items = (long long)pairs * (g.ny - 2);
+    const dim3 grid((unsigned)((items + BX * BY - 1) / (BX * BY)),
+                    (unsigned)((g.nz - 2 + kRefZ - 1) / kRefZ));
+    hipLaunchKernelGGL(k_rbsor_half, grid, dim3(BX, BY), 0, st, g, p, d, flags, colour, omega,
+                       pairs);
+    return hipGetLastError();
+}
+
 hipError_t rbsor_sweeps(const Grid& g, float* const (&p)[2], int* cur, const float* d,
                         const uint8_t* flags, int sweeps, float omega, int cold, hipStream_t st,
                         int* launches)
 {
-    // 4 or 6 half-sweeps per launch, whichever takes fewer steps per
-    // half-sweep; narrow columns where the grid is too small to fill the CUs
-    // with wide ones.  us per half-sweep, narrow 4 / 4 / 6: 48x40x57 2.1 / 2.8
-    // / 2.7, 80^3 2.6 / 2.9 / 2.8, 113x90x101 3.2 / 3.3 / 3.4, 150^3 4.8 / 5.0 /
-    // 4.7, 256x240x248 13.3 / 12.3 / 11.8.
-    const bool narrow = (long long)g.nx * g.ny * g.nz <= 1500000;
-    const int H = narrow || pressure_plan<32, 4>(g).steps * 6 <= pressure_plan<32, 6>(g).steps * 4 ? 4 : 6;
-    const int n = (sweeps + H - 1) / H;
+    const PressureRoute r = pressure_route(g);
+    const int n = (sweeps + r.H - 1) / r.H;
     *launches = 0;
     for (int l = 0, done = 0; l < n; ++l) {
         const int m = sweeps / n + (l < sweeps % n ? 1 : 0), colour = done & 1;
@@ -884,9 +981,10 @@ hipError_t rbsor_sweeps(const Grid& g, float* const (&p)[2], int* cur, const flo
         float* po = p[*cur ^ 1];
         const int zero_in = cold && l == 0;
         const hipError_t e =
-            narrow   ? launch_pressure_march<16, 4>(g, pi, po, d, flags, colour, m, omega, zero_in, st)
-            : H == 4 ? launch_pressure_march<32, 4>(g, pi, po, d, flags, colour, m, omega, zero_in, st)
-                     : launch_pressure_march<32, 6>(g, pi, po, d, flags, colour, m, omega, zero_in, st);
+            r.narrow ? launch_pressure_march<16, 4>(g, r.plan, pi, po, d, flags, colour, m, omega, zero_in, st)
+            : r.H == 4
+                ? launch_pressure_march<32, 4>(g, r.plan, pi, po, d, flags, colour, m, omega, zero_in, st)
+                : launch_pressure_march<32, 6>(g, r.plan, pi, po, d, flags, colour, m, omega, zero_in, st);
         if (e != hipSuccess) return e;
         *cur ^= 1;
         done += m;

@@ -446,6 +446,24 @@ def case_thin_reference():
         g.close()
 
 
+def case_thin_pressure():
+    # The same for the pressure form, cold and warm; the pressure changes
+    # buffers or not by the route.
+    for dims, its, warm, several in [((60, 3, 1500), 3, 1, False), ((60, 3, 1500), 2, 0, False),
+                                     ((14, 12, 10), 3, 1, True)]:
+        sc = scenes.test_scene(dims, seed=39, projection=1, iterations=its, box_fraction=0.0,
+                               n_obstacles=0)
+        sc["params"]["warm_start"] = warm
+        g, o = gpu_for(sc), oracle_for(sc, 32)
+        n = _sweep_launches(g, sc["dt"])
+        assert (n < 2 * its) == several, (dims, its, n)
+        g.step(sc["dt"], readback=False)
+        o.step(sc["dt"], 2)
+        assert_bitwise_equal(g.state(), o.state(), f"thin {dims} x{its} warm {warm}")
+        same_bits(g.get_pressure(), o.get_pressure(), f"thin {dims} x{its} warm {warm}")
+        g.close()
+
+
 def case_foreign_capture():
     # A first step of the reference form while another stream is captured in
     # the global mode: the capture goes on, and this and later steps run
@@ -467,7 +485,7 @@ def case_foreign_capture():
     g.close()
 
 
-CASES = {"thin_reference": case_thin_reference, "read_slots": case_read_slots, "small_reads": case_small_reads, "foreign_capture": case_foreign_capture, "read_targets": case_read_targets, "step_graph": case_step_graph, "proxy": case_proxy, "refine_groups": case_refine_groups, "single": case_single, "norms": case_norms, "plans": case_plans, "batch": case_batch,
+CASES = {"thin_pressure": case_thin_pressure, "thin_reference": case_thin_reference, "read_slots": case_read_slots, "small_reads": case_small_reads, "foreign_capture": case_foreign_capture, "read_targets": case_read_targets, "step_graph": case_step_graph, "proxy": case_proxy, "refine_groups": case_refine_groups, "single": case_single, "norms": case_norms, "plans": case_plans, "batch": case_batch,
          "server": case_server, "readback": case_readback, "precision": case_precision,
          "vorticity": case_vorticity, "advection": case_advection}
 
