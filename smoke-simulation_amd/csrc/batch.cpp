@@ -613,35 +613,40 @@ smoke_status smoke_batch_autotune(smoke_batch* b, smoke_jacobi_plan* chosen, dou
     hipEvent_t ev[2];
     HIP_TRY(hipEventCreate(&ev[0]));
     HIP_TRY(hipEventCreate(&ev[1]));
-    smk::JacobiPlan best = b->plan;
+    const smk::JacobiPlan given = b->plan;
+    smk::JacobiPlan best = given;
     double best_ms = -1.0;
     const int tiles[4] = {smk::JacobiPlan::TILE_32x32, smk::JacobiPlan::TILE_64x16,
                           smk::JacobiPlan::TILE_64x32, smk::JacobiPlan::TILE_32x64};
-    const int zcs[4] = {32, 64, 128, 256};
+    // Short chunks too: a small batch occupies few CUs with long ones.
+    const int zcs[6] = {8, 16, 32, 64, 128, 256};
     hipError_t e = hipSuccess;
+    auto time = [&](int t, int tile, int zc) {
+        b->plan.sweeps_per_launch = t;
+        b->plan.tile = tile;
+        b->plan.zc = std::min(zc, b->zc_cap);
+        e = rebuild_jacobi_table(b);
+        int L = 0;
+        if (e == hipSuccess) e = enqueue_sweeps(b, b->plan, &L);  // warm-up
+        if (e == hipSuccess) e = hipEventRecord(ev[0], b->stream);
+        for (int r = 0; r < 2 && e == hipSuccess; ++r) e = enqueue_sweeps(b, b->plan, &L);
+        if (e == hipSuccess) e = hipEventRecord(ev[1], b->stream);
+        if (e == hipSuccess) e = hipEventSynchronize(ev[1]);
+        float ms = 0.0f;
+        if (e == hipSuccess) e = hipEventElapsedTime(&ms, ev[0], ev[1]);
+        if (e != hipSuccess) return;
+        const double per = ms / (2.0 * b->iterations);
+        if (best_ms < 0.0 || per < best_ms) {
+            best_ms = per;
+            best = b->plan;
+        }
+    };
+    // The plan in force (fitted or given) first: another has to be faster.
+    time(given.sweeps_per_launch, given.tile, given.zc);
     for (int t = 2; t <= 6 && e == hipSuccess; ++t)
         for (int tile : tiles)
-            for (int zc : zcs) {
-                if (e != hipSuccess) break;  // a failed candidate ends the search
-                b->plan.sweeps_per_launch = t;
-                b->plan.tile = tile;
-                b->plan.zc = std::min(zc, b->zc_cap);
-                e = rebuild_jacobi_table(b);
-                int L = 0;
-                if (e == hipSuccess) e = enqueue_sweeps(b, b->plan, &L);  // warm-up
-                if (e == hipSuccess) e = hipEventRecord(ev[0], b->stream);
-                for (int r = 0; r < 2 && e == hipSuccess; ++r) e = enqueue_sweeps(b, b->plan, &L);
-                if (e == hipSuccess) e = hipEventRecord(ev[1], b->stream);
-                if (e == hipSuccess) e = hipEventSynchronize(ev[1]);
-                float ms = 0.0f;
-                if (e == hipSuccess) e = hipEventElapsedTime(&ms, ev[0], ev[1]);
-                if (e != hipSuccess) break;
-                const double per = ms / (2.0 * b->iterations);
-                if (best_ms < 0.0 || per < best_ms) {
-                    best_ms = per;
-                    best = b->plan;
-                }
-            }
+            for (int zc : zcs)
+                if (e == hipSuccess) time(t, tile, zc);  // a failed candidate ends the search
     (void)hipEventDestroy(ev[0]);
     (void)hipEventDestroy(ev[1]);
     b->plan = b->reported = best;

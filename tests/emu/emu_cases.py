@@ -430,6 +430,30 @@ def _sweep_launches(g, dt):
     return n
 
 
+def case_batch_autotune():
+    # Every candidate takes the same time here: the plan in force, fitted or
+    # given, stays.
+    scs = [scenes.test_scene(d, seed=50 + k, projection=2, iterations=1, n_obstacles=0)
+           for k, d in enumerate([(12, 10, 9), (9, 12, 20)])]
+    for given in (None, dict(sweeps_per_launch=3, tile=1, zc=5)):
+        sims = [gpu_for(sc) for sc in scs]
+        b = smokesim.Batch(sims, [0.05, 0.05])
+        if given:
+            b.set_jacobi_plan(**given)
+        plan, _ = b.autotune()
+        assert plan == (given or dict(sweeps_per_launch=5, tile=0, zc=plan["zc"])), plan
+        assert plan["zc"] < 32 and b.get_jacobi_plan() == plan, plan
+        b.step(use_graph=False)
+        b.synchronize()
+        for sc, g in zip(scs, sims):
+            o = oracle_for(sc, 32)
+            o.step(0.05, 1)
+            assert_bitwise_equal(g.state(), o.state(), f"{sc['name']} {plan}")
+        b.close()
+        for g in sims:
+            g.close()
+
+
 def case_thin_reference():
     # Grids whose columns would be mostly empty run one half-sweep per launch,
     # others several, with the same bits; a change of the iteration count may
@@ -485,7 +509,7 @@ def case_foreign_capture():
     g.close()
 
 
-CASES = {"thin_pressure": case_thin_pressure, "thin_reference": case_thin_reference, "read_slots": case_read_slots, "small_reads": case_small_reads, "foreign_capture": case_foreign_capture, "read_targets": case_read_targets, "step_graph": case_step_graph, "proxy": case_proxy, "refine_groups": case_refine_groups, "single": case_single, "norms": case_norms, "plans": case_plans, "batch": case_batch,
+CASES = {"batch_autotune": case_batch_autotune, "thin_pressure": case_thin_pressure, "thin_reference": case_thin_reference, "read_slots": case_read_slots, "small_reads": case_small_reads, "foreign_capture": case_foreign_capture, "read_targets": case_read_targets, "step_graph": case_step_graph, "proxy": case_proxy, "refine_groups": case_refine_groups, "single": case_single, "norms": case_norms, "plans": case_plans, "batch": case_batch,
          "server": case_server, "readback": case_readback, "precision": case_precision,
          "vorticity": case_vorticity, "advection": case_advection}
 

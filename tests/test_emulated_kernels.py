@@ -63,7 +63,8 @@ def test_emulated_case_with_deferred_streams(emu_lib, case):
 @pytest.mark.parametrize("case,deferred", [("read_targets", False), ("read_targets", True),
                                            ("foreign_capture", False), ("small_reads", False),
                                            ("read_slots", False), ("read_slots", True),
-                                           ("thin_reference", False), ("thin_pressure", False)])
+                                           ("thin_reference", False), ("thin_pressure", False),
+                                           ("batch_autotune", False)])
 def test_emulated_host_path(emu_lib, case, deferred):
     """What the host code asks of the runtime (tests/emu/emu_cases.py)."""
     lib, asan = emu_lib
