@@ -157,7 +157,12 @@ void smoke_destroy(smoke_sim* sim);
 
 smoke_status smoke_get_dims(const smoke_sim* sim, unsigned* nx, unsigned* ny, unsigned* nz);
 
-/* Device bytes held by one simulation of the given size (budgeting). */
+/* Device bytes held by one simulation of the given size (budgeting).  What has
+ * buffers of its own takes them on first use: vorticity (four FP32 fields),
+ * obstacle_velocity (a byte per cell), step norms, the asynchronous read-back
+ * (two density arrays), and the REFERENCE projection of a simulation that has run
+ * a pressure form, was restored or has step norms on (three FP32 fields, if the
+ * device has them: its steps are slower without, with the same results). */
 size_t smoke_footprint_bytes(unsigned nx, unsigned ny, unsigned nz);
 /* ... with a storage and, if `refined`, the REFINED solver's buffers. */
 size_t smoke_footprint_bytes_ex(unsigned nx, unsigned ny, unsigned nz, int storage, int refined);

@@ -420,7 +420,8 @@ smoke_status smoke_batch_create(smoke_sim* const* sims, int count, const float* 
     // simulations' own streams finished.
     for (smoke_sim* s : b->sims) {
         std::lock_guard<std::mutex> lk(s->mu);
-        if (smk::refresh_mask(s, nullptr) != hipSuccess || hipStreamSynchronize(s->stream) != hipSuccess)
+        if (smk::refresh_mask(s, nullptr) != hipSuccess || smk::reclaim_scratch(s) != hipSuccess ||
+            hipStreamSynchronize(s->stream) != hipSuccess)
             return bail(fail(SMOKE_ERR_HIP, "batch_create: preparing a simulation failed"));
     }
     // Descriptors.
@@ -497,6 +498,7 @@ smoke_status smoke_batch_create(smoke_sim* const* sims, int count, const float* 
         std::lock_guard<std::mutex> lk(s->mu);
         s->batch = b;
         s->batch_stream = b->stream;
+        s->pressure_kept = true;
     }
     *out = b;
     return SMOKE_OK;

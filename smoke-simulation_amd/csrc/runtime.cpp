@@ -183,6 +183,17 @@ hipError_t smk::refresh_mask(smoke_sim* s, long long* launches)
     return hipSuccess;
 }
 
+hipError_t smk::reclaim_scratch(smoke_sim* s)
+{
+    if (!s->scratch_dirty) return hipSuccess;
+    for (float* f : {s->P[0], s->P[1], s->d}) {
+        const hipError_t e = smk::fill_f32(f, s->g.elems, 0.0f, s->stream);
+        if (e != hipSuccess) return e;
+    }
+    s->scratch_dirty = false;
+    return hipSuccess;
+}
+
 namespace {
 
 // Allocates and clears the REFINED buffers (once per simulation).
@@ -259,23 +270,35 @@ struct AllowWhileCapturing {
     ~AllowWhileCapturing() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
 };
 
-// Allocates the reference projection's second velocity set (once per
-// simulation, before a step or a capture of its own, where its launches are
-// the faster ones).  They write every entry they later read.
-void ensure_sweep_fields(smoke_sim* s)
+// Whether the reference projection's launches may use P and d as their second
+// velocity set: a simulation that never ran a pressure form holds nothing in
+// them, and zeros are what reclaim_scratch puts back.
+bool arena_scratch(const smoke_sim* s) { return !s->pressure_kept && !s->norms_on; }
+
+// Before the projection is enqueued (and outside a capture of the simulation's
+// own): the fields it needs.  For the reference form whose P or d are taken
+// that is a set of its own, allocated once.  Its launches write every entry
+// they later read.
+hipError_t prepare_project(smoke_sim* s)
 {
-    if (s->prm.projection != SMOKE_PROJ_REFERENCE || s->sweep_mem || s->sweep_refused ||
+    const bool reference = s->prm.projection == SMOKE_PROJ_REFERENCE;
+    if (!reference || !arena_scratch(s)) {
+        const hipError_t e = smk::reclaim_scratch(s);
+        if (e != hipSuccess) return e;
+    }
+    if (!reference || arena_scratch(s) || s->sweep_mem || s->sweep_refused ||
         smk::reference_in_place(s->g, 2 * s->prm.iterations))
-        return;
+        return hipSuccess;
     const AllowWhileCapturing allow;
     const size_t field = align256((size_t)s->g.elems * sizeof(float));
     if (hipMalloc((void**)&s->sweep_mem, 3 * field) != hipSuccess) {
         smk::forget_last_error();  // the launches' checks must not find it
         s->sweep_mem = nullptr;
         s->sweep_refused = true;
-        return;
+        return hipSuccess;
     }
     for (int k = 0; k < 3; ++k) s->sweep_vel[k] = reinterpret_cast<float*>(s->sweep_mem + k * field);
+    return hipSuccess;
 }
 
 // Allocates the step-norms records (once per simulation): the reduction's
@@ -461,10 +484,14 @@ hipError_t stage_project(smoke_sim* s, long long* launches)
         }
         if ((e = sweep_mark(s, 0, 0)) != hipSuccess) return e;
         int n_launches = 2 * p.iterations;
-        if (s->sweep_mem && !smk::reference_in_place(g, n_launches)) {
+        const bool scratch = arena_scratch(s);
+        if ((scratch || s->sweep_mem) && !smk::reference_in_place(g, n_launches)) {
             float* const vel[3] = {s->u[n], s->v[n], s->w[n]};
-            e = smk::project_reference_sweeps(g, vel, s->sweep_vel, s->flags, 2 * p.iterations,
-                                              p.sor_omega, s->stream, &n_launches);
+            float* other[3] = {s->P[0], s->P[1], s->d};
+            if (!scratch) std::copy(s->sweep_vel, s->sweep_vel + 3, other);
+            s->scratch_dirty = s->scratch_dirty || scratch;
+            e = smk::project_reference_sweeps(g, vel, other, s->flags, n_launches, p.sor_omega, s->stream,
+                                              &n_launches);
             if (e != hipSuccess) return e;
         } else {
             for (int k = 0; k < n_launches; ++k) {
@@ -476,6 +503,7 @@ hipError_t stage_project(smoke_sim* s, long long* launches)
         *launches += n_launches;
         return sweep_mark(s, 1, n_launches);
     }
+    s->pressure_kept = true;
     e = smk::with_fields(s, [&](auto, auto u, auto v, auto w) {
         return smk::divergence(g, u[n], v[n], w[n], s->flags, s->d, s->stream);
     });
@@ -647,7 +675,8 @@ smoke_status step_graph(smoke_sim* s, float dt)
         if (sg.graph) (void)hipGraphDestroy(sg.graph);
         sg = smoke_sim::StepGraph{};
         const int now0 = s->now, pcur0 = s->pcur;
-        const bool rhs0 = s->rhs_valid;
+        const bool rhs0 = s->rhs_valid, dirty0 = s->scratch_dirty;
+        s->scratch_dirty = false;
         HIP_TRY(hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal));
         hipError_t e = hipSuccess;
         for (int st = 0; st < SMOKE_STAGE_COUNT && e == hipSuccess; ++st) {
@@ -659,6 +688,8 @@ smoke_status step_graph(smoke_sim* s, float dt)
         sg.now_out = s->now;
         sg.pcur_out = s->pcur;
         sg.rhs_out = s->rhs_valid;
+        sg.scratch = s->scratch_dirty;
+        s->scratch_dirty = dirty0;
         s->now = now0;  // the replay below applies the step's parities
         s->pcur = pcur0;
         s->rhs_valid = rhs0;
@@ -683,6 +714,7 @@ smoke_status step_graph(smoke_sim* s, float dt)
     s->now = sg.now_out;
     s->pcur = sg.pcur_out;
     s->rhs_valid = sg.rhs_out;
+    s->scratch_dirty = s->scratch_dirty || sg.scratch;
     s->last_dt = dt;
     s->steps_enqueued += 1;
     return SMOKE_OK;
@@ -692,7 +724,7 @@ smoke_status step_locked(smoke_sim* s, float dt)
 {
     SMOKE_REFUSE_IN_BATCH(s, "step");
     if (!std::isfinite(dt)) return fail(SMOKE_ERR_INVALID, "step: dt must be finite");
-    ensure_sweep_fields(s);
+    HIP_TRY(prepare_project(s));
     if (s->graph_on && !s->timing && !s->norms_on) return step_graph(s, dt);
     smoke_sim::StepEvents se{};
     if (s->timing) {
@@ -1189,6 +1221,7 @@ smoke_status smoke_snapshot(smoke_sim* s, void* host, size_t bytes)
     const size_t need = snapshot_size(s, s->objects.size());
     if (bytes < need) return fail(SMOKE_ERR_INVALID, "snapshot: buffer holds %zu bytes, needs %zu", bytes, need);
     SMOKE_WAIT_BATCH(s);
+    HIP_TRY(smk::reclaim_scratch(s));
     HIP_TRY(hipStreamSynchronize(s->stream));
     SnapshotHeader h;
     std::memset(&h, 0, sizeof h);
@@ -1260,6 +1293,8 @@ smoke_status smoke_restore(smoke_sim* s, const void* host, size_t bytes)
     s->now = h.now;
     s->pcur = h.pcur;
     s->prm = h.prm;
+    s->pressure_kept = true;  // as far as known
+    s->scratch_dirty = false;
     s->plan.sweeps_per_launch = h.plan[0];
     s->plan.tile = h.plan[1];
     s->plan.zc = h.plan[2];
@@ -1320,6 +1355,7 @@ smoke_status smoke_autotune(smoke_sim* s, smoke_jacobi_plan* chosen, double* ms_
     SMOKE_REFUSE_IN_BATCH(s, "autotune");
     const int K = s->prm.iterations > 0 ? s->prm.iterations : 100;
     HIP_TRY(refresh_mask(s, nullptr));
+    HIP_TRY(smk::reclaim_scratch(s));
     hipEvent_t ev[2] = {nullptr, nullptr};
     auto cleanup = [&]() {
         for (hipEvent_t e : ev)
@@ -1596,6 +1632,7 @@ smoke_status smoke_get_pressure(smoke_sim* s, float* dst)
 {
     if (!s || !dst) return fail(SMOKE_ERR_INVALID, "get_pressure: NULL");
     std::lock_guard<std::mutex> lk(s->mu);
+    HIP_TRY(smk::reclaim_scratch(s));
     return read_cells_f32(s, s->P[s->pcur], dst);
 }
 
@@ -1642,7 +1679,7 @@ smoke_status smoke_run_stage(smoke_sim* s, int stage, float dt)
     SMOKE_REFUSE_IN_BATCH(s, "run_stage");
     s->norms_step = -1;
     s->last_dt = dt;
-    ensure_sweep_fields(s);
+    if (stage == SMOKE_STAGE_PROJECT) HIP_TRY(prepare_project(s));
     long long launches = 0;
     hipError_t e = run_stage(s, stage, dt, &launches);
     if (e != hipSuccess) return fail(SMOKE_ERR_HIP, "run_stage %d: %s", stage, hipGetErrorString(e));

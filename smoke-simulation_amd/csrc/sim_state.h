@@ -64,9 +64,15 @@ struct smoke_sim {
     // above 0).
     char* vort_mem = nullptr;
     smk::VortBufs vb{};
-    // Second set of velocity fields of the reference projection's half-sweeps
-    // (allocated before the first step that uses them; without memory for
-    // them, sweep_refused, the half-sweeps run in place, one per launch).
+    // P, after a pressure form: the last solve's result (get_pressure, warm
+    // starts).  Until then P and d are zero and serve the reference projection as
+    // its second set of velocity fields; scratch_dirty: they hold that set's
+    // entries, to be cleared before any other use (smk::reclaim_scratch).
+    bool pressure_kept = false;
+    bool scratch_dirty = false;
+    // That set where P or d are taken (allocated before the first such step;
+    // without memory for it, sweep_refused, the half-sweeps run in place, one per
+    // launch).
     char* sweep_mem = nullptr;
     bool sweep_refused = false;
     float* sweep_vel[3] = {nullptr, nullptr, nullptr};
@@ -126,6 +132,7 @@ struct smoke_sim {
         float dt = 0.0f;
         int pcur_in = -1, now_out = 0, pcur_out = 0;
         bool rhs_out = false;
+        bool scratch = false;  // the step leaves scratch_dirty
     };
     bool graph_on = false;
     unsigned long long version = 1;
@@ -172,6 +179,9 @@ auto with_fields(smoke_sim* s, Fn&& fn)
 hipError_t enqueue_norms(smoke_sim* s, void* scratch, smoke_step_norms* out);
 // Rebuilds mask and flags if the base mask or an obstacle changed.
 hipError_t refresh_mask(smoke_sim* s, long long* launches);
+// Clears P and d (on the simulation's stream) if the reference projection used
+// them; before anything else reads or relies on them.
+hipError_t reclaim_scratch(smoke_sim* s);
 // Called by smoke_destroy for a simulation that is still in a batch: waits
 // for the batch and marks it unusable (its steps would touch freed memory).
 void batch_detach(smoke_batch* b, smoke_sim* s);

@@ -454,6 +454,83 @@ def case_batch_autotune():
             g.close()
 
 
+def _same_state(g, o, what):
+    assert_bitwise_equal(g.state(), o.state(), what)
+    same_bits(g.get_pressure(), o.get_pressure(), what + " pressure")
+
+
+def case_reference_memory():
+    # The reference form holds no more than the footprint: its half-sweeps use
+    # the pressure form's fields, which are zero again for everything that reads
+    # them.
+    dims, its = (14, 12, 10), 4
+    fp = smokesim.footprint_bytes(*dims)
+
+    def both(seed, **kw):
+        sc = scenes.test_scene(dims, seed=seed, projection=0, iterations=its, **kw)
+        return sc, gpu_for(sc), oracle_for(sc, 32)
+
+    def step(sc, g, o, n=1):
+        for _ in range(n):
+            g.step(sc["dt"], readback=False)
+        o.step(sc["dt"], n)
+
+    def change(g, o, **kw):
+        for s in (g, o):
+            s.set_params(**kw)
+
+    for graph in (False, True):
+        sc, g, o = both(60)
+        assert _emu("emu_device_bytes") == fp
+        g.set_step_graph(graph)
+        assert _sweep_launches(g, sc["dt"]) < 2 * its
+        o.step(sc["dt"], 1)
+        step(sc, g, o, 3)
+        assert _emu("emu_device_bytes") == fp
+        _same_state(g, o, f"graph {graph}")           # the pressure is still zero
+        step(sc, g, o, 2)                             # (a replay after it was cleared)
+        blob = g.snapshot()
+        step(sc, g, o)
+        r = gpu_for(sc)
+        r.restore(blob)
+        r.step(sc["dt"], readback=False)
+        _same_state(r, o, f"restored, graph {graph}")
+        r.close()
+        for proj, warm in ((2, 0), (1, 1), (2, 1), (0, 0), (1, 1)):
+            change(g, o, projection=proj, warm_start=warm)
+            step(sc, g, o, 2)
+            _same_state(g, o, f"then projection {proj}, graph {graph}")
+        g.close()
+    # Warm from the zero pressure; norms, whose right-hand side is kept; a batch.
+    sc, g, o = both(61, noise=0.4)
+    step(sc, g, o)
+    change(g, o, projection=1, warm_start=1)
+    step(sc, g, o)
+    _same_state(g, o, "warm after reference")
+    g.close()
+    import oracle as orc
+    sc, g, o = both(62, noise=0.4)
+    step(sc, g, o)
+    g.norms_enable(True)
+    step(sc, g, o)
+    n, m = g.step_norms(), orc.step_norms(g, sc["dt"])
+    assert n["rhs_l2"] > n["div_l2"] and abs(n["div_l2"] - m["div_l2"]) <= 1e-12 * m["div_l2"]
+    g.norms_enable(False)
+    step(sc, g, o, 2)
+    _same_state(g, o, "norms")
+    change(g, o, projection=2)
+    b = smokesim.Batch([g], [sc["dt"]])
+    for _ in range(2):
+        b.step(use_graph=False)
+    b.close()
+    o.step(sc["dt"], 2)
+    _same_state(g, o, "batch")
+    change(g, o, projection=0)
+    step(sc, g, o, 2)
+    _same_state(g, o, "after the batch")
+    g.close()
+
+
 def case_thin_reference():
     # Grids whose columns would be mostly empty run one half-sweep per launch,
     # others several, with the same bits; a change of the iteration count may
@@ -496,20 +573,32 @@ def case_foreign_capture():
     sc = scenes.test_scene((14, 12, 10), seed=36, projection=0, iterations=6)
     g, o = gpu_for(sc), oracle_for(sc, 32)
     hip = smokesim.load()
-    st, graph = ctypes.c_void_p(), ctypes.c_void_p()
-    assert hip.hipStreamCreateWithFlags(ctypes.byref(st), 1) == 0
-    assert hip.hipStreamBeginCapture(st, 0) == 0
+
+    def captured_step():
+        st, graph = ctypes.c_void_p(), ctypes.c_void_p()
+        assert hip.hipStreamCreateWithFlags(ctypes.byref(st), 1) == 0
+        assert hip.hipStreamBeginCapture(st, 0) == 0
+        g.step(sc["dt"], readback=False)
+        assert hip.hipStreamEndCapture(st, ctypes.byref(graph)) == 0
+        assert hip.hipGraphDestroy(graph) == 0 and hip.hipStreamDestroy(st) == 0
+
+    captured_step()
+    assert _sweep_launches(g, sc["dt"]) < 2 * 6
+    o.step(sc["dt"], 2)
+    for s in (g, o):
+        s.set_params(projection=2)  # after it the reference form has a set of its own
     g.step(sc["dt"], readback=False)
-    assert hip.hipStreamEndCapture(st, ctypes.byref(graph)) == 0
-    assert hip.hipGraphDestroy(graph) == 0 and hip.hipStreamDestroy(st) == 0
-    n = _sweep_launches(g, sc["dt"])
-    assert n < 2 * 6, n
+    o.step(sc["dt"], 1)
+    for s in (g, o):
+        s.set_params(projection=0)
+    captured_step()
+    assert _sweep_launches(g, sc["dt"]) < 2 * 6
     o.step(sc["dt"], 2)
     assert_bitwise_equal(g.state(), o.state(), "foreign capture")
     g.close()
 
 
-CASES = {"batch_autotune": case_batch_autotune, "thin_pressure": case_thin_pressure, "thin_reference": case_thin_reference, "read_slots": case_read_slots, "small_reads": case_small_reads, "foreign_capture": case_foreign_capture, "read_targets": case_read_targets, "step_graph": case_step_graph, "proxy": case_proxy, "refine_groups": case_refine_groups, "single": case_single, "norms": case_norms, "plans": case_plans, "batch": case_batch,
+CASES = {"reference_memory": case_reference_memory, "batch_autotune": case_batch_autotune, "thin_pressure": case_thin_pressure, "thin_reference": case_thin_reference, "read_slots": case_read_slots, "small_reads": case_small_reads, "foreign_capture": case_foreign_capture, "read_targets": case_read_targets, "step_graph": case_step_graph, "proxy": case_proxy, "refine_groups": case_refine_groups, "single": case_single, "norms": case_norms, "plans": case_plans, "batch": case_batch,
          "server": case_server, "readback": case_readback, "precision": case_precision,
          "vorticity": case_vorticity, "advection": case_advection}
 

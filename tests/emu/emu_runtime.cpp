@@ -338,6 +338,7 @@ hipError_t hipMalloc(void** p, size_t n)
 {
     Lock lk(g_mu);
     if (unsafe_call()) return hipErrorStreamCaptureUnsupported;
+    if (n > g_refuse_above) return hipErrorOutOfMemory;
     *p = malloc(n ? n : 1);
     g_device[*p] = n;
     return hipSuccess;
@@ -563,10 +564,16 @@ hipError_t hipEventElapsedTime(float* ms, hipEvent_t a, hipEvent_t b)
 }
 
 // What a test asks of the emulator: pinned allocations asked for so far and
-// held now, the asynchronous copies into the device allocation at `base`; and
-// to refuse allocations of more than n bytes.
+// held now, the device bytes held, the asynchronous copies into the device
+// allocation at `base`; and to refuse allocations of more than n bytes.
 long long emu_pinned_calls() { return g_pinned_calls; }
 long long emu_pinned_held() { return (long long)g_pinned.size(); }
+long long emu_device_bytes()
+{
+    long long n = 0;
+    for (const auto& a : g_device) n += (long long)a.second;
+    return n;
+}
 void emu_refuse_above(size_t n) { g_refuse_above = n; }
 long long emu_copies_into(void* base)
 {
