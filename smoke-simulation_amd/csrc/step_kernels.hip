@@ -745,24 +745,30 @@ static FacesRoute faces_route(const Grid& g)
 // An even number of launches, so that the last one writes the first set again.
 static int faces_launches(const FacesRoute& r, int sweeps) { return 2 * ((sweeps + 2 * r.H - 1) / (2 * r.H)); }
 
+// The 128-byte lines of a field that a half-sweep visits.
+static double half_sweep_lines(const Grid& g) { return (double)(g.ny - 2) * (g.nz - 2) * ((g.nx + 31) / 32); }
+static double interior_cells(const Grid& g) { return (double)(g.nx - 2) * (g.ny - 2) * (g.nz - 2); }
+
 // A column of the marched launches costs the same however few of its cells the
 // grid has, and a grid thin in x or y fills little of it: one half-sweep per
 // launch in place is then faster.  Both by their measured times (400 random
-// grids, extents 3..20000, within 5 % for most): a marched launch 2.5 us and 1.1
-// a step, a half-sweep 2.8 us, 6.9 per 10^5 128-byte lines and 3.4 per 10^6
-// cells.  The march has to gain 15 % by these.  us for 40 half-sweeps, in place /
+// grids, extents 3..20000, within 5 % for most): a marched launch 2.5 us, and 0.6
+// and 0.125 for each half-sweep a step; a half-sweep 2.8 us, 6.9 per 10^5
+// 128-byte lines and 3.4 per 10^6 cells.  The march has to gain 15 % by these.
+// us for 40 half-sweeps, in place /
 // marched: 18072x3x56 290 / 1290, 59x4x19372 569 / 1864, 10x4x3220 146 / 299,
 // 129x9x882 249 / 282, 130x3308x6 388 / 412; 28x120x289 326 / 226, 150x96x121
-// 431 / 226.
+// 431 / 226 (4 of them 43 / 34).  Of the boxes' two launches, 4 half-sweeps in
+// place are faster or as fast: 16x16x40 12 / 15, 80^3 21 / 21.
 bool reference_in_place(const Grid& g, int sweeps)
 {
     if (sweeps < 4) return true;
     if ((g.nz - 2 + kRefZ - 1) / kRefZ > 65535) return false;  // a grid's y extent
     const FacesRoute r = faces_route(g);
-    if (r.boxed) return false;
-    const double rows = (double)(g.ny - 2) * (g.nz - 2), lines = rows * ((g.nx + 31) / 32);
-    const double in_place = sweeps * (2.8 + 6.9e-5 * lines + 3.4e-6 * rows * (g.nx - 2));
-    return in_place < 1.15 * faces_launches(r, sweeps) * (2.5 + 1.1 * (double)r.plan.steps);
+    if (r.boxed) return sweeps < 6;
+    const double in_place = sweeps * (2.8 + 6.9e-5 * half_sweep_lines(g) + 3.4e-6 * interior_cells(g));
+    const int n = faces_launches(r, sweeps);
+    return in_place < 1.15 * n * (2.5 + (0.6 + 0.125 * sweeps / n) * (double)r.plan.steps);
 }
 
 hipError_t project_reference_sweeps(const Grid& g, float* const (&a)[3], float* const (&b)[3],
@@ -949,8 +955,8 @@ bool rbsor_in_place(const Grid& g, int sweeps)
     if (sweeps == 0) return true;
     if ((g.nz - 2 + kRefZ - 1) / kRefZ > 65535) return false;  // a grid's y extent
     const PressureRoute r = pressure_route(g);
-    const double rows = (double)(g.ny - 2) * (g.nz - 2), lines = rows * ((g.nx + 31) / 32);
-    const double in_place = sweeps * (2.35 + 4.2e-5 * lines + 2.3e-6 * rows * (g.nx - 2)) + 2.3 + 1e-6 * g.elems;
+    const double in_place = sweeps * (2.35 + 4.2e-5 * half_sweep_lines(g) + 2.3e-6 * interior_cells(g)) +
+                            2.3 + 1e-6 * g.elems;
     const bool shared = (long long)r.plan.grid.x * r.plan.grid.y * r.plan.grid.z > kCUs;
     const double step = r.narrow ? (shared ? 0.39 : 0.535) : 0.86;
     return in_place < 1.1 * sweeps / r.H * (2.5 + step * (double)r.plan.steps);
