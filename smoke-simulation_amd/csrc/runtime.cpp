@@ -1183,6 +1183,7 @@ smoke_status smoke_set_params(smoke_sim* s, const smoke_params* p)
         if (os != SMOKE_OK) return os;
     }
     s->prm = *p;
+    s->sweep_refused = false;
     s->version += 1;
     return SMOKE_OK;
 }
@@ -1295,6 +1296,7 @@ smoke_status smoke_restore(smoke_sim* s, const void* host, size_t bytes)
     s->prm = h.prm;
     s->pressure_kept = true;  // as far as known
     s->scratch_dirty = false;
+    s->sweep_refused = false;
     s->plan.sweeps_per_launch = h.plan[0];
     s->plan.tile = h.plan[1];
     s->plan.zc = h.plan[2];

@@ -72,7 +72,7 @@ struct smoke_sim {
     bool scratch_dirty = false;
     // That set where P or d are taken (allocated before the first such step;
     // without memory for it, sweep_refused, the half-sweeps run in place, one per
-    // launch).
+    // launch, until the parameters are set again).
     char* sweep_mem = nullptr;
     bool sweep_refused = false;
     float* sweep_vel[3] = {nullptr, nullptr, nullptr};

@@ -531,6 +531,42 @@ def case_reference_memory():
     g.close()
 
 
+def case_refused_set():
+    # Without memory for the reference form's own velocity set (after a pressure
+    # form) its steps run in place with the same bits; setting the parameters
+    # again asks again.
+    sc = scenes.test_scene((14, 12, 10), seed=64, projection=2, iterations=4)
+    g, o = gpu_for(sc), oracle_for(sc, 32)
+
+    def step(**kw):
+        for s in (g, o):
+            s.set_params(**kw)
+        o.step(sc["dt"], 1)
+        return _sweep_launches(g, sc["dt"])
+
+    step()
+    _emu("emu_refuse_above", 1000)
+    assert step(projection=0) == 8
+    o.step(sc["dt"], 1)
+    assert _sweep_launches(g, sc["dt"]) == 8
+    _same_state(g, o, "refused")
+    _emu("emu_refuse_above", 2 ** 63)
+    assert step(iterations=5) < 10
+    blob = g.snapshot()
+    _same_state(g, o, "allocated")
+    r = gpu_for(sc)
+    _emu("emu_refuse_above", 1000)
+    r.restore(blob)
+    assert _sweep_launches(r, sc["dt"]) == 10
+    _emu("emu_refuse_above", 2 ** 63)
+    r.restore(blob)
+    assert _sweep_launches(r, sc["dt"]) < 10
+    o.step(sc["dt"], 1)
+    _same_state(r, o, "restored")
+    r.close()
+    g.close()
+
+
 def case_thin_reference():
     # Grids whose columns would be mostly empty run one half-sweep per launch,
     # others several, with the same bits; a change of the iteration count may
@@ -598,7 +634,7 @@ def case_foreign_capture():
     g.close()
 
 
-CASES = {"reference_memory": case_reference_memory, "batch_autotune": case_batch_autotune, "thin_pressure": case_thin_pressure, "thin_reference": case_thin_reference, "read_slots": case_read_slots, "small_reads": case_small_reads, "foreign_capture": case_foreign_capture, "read_targets": case_read_targets, "step_graph": case_step_graph, "proxy": case_proxy, "refine_groups": case_refine_groups, "single": case_single, "norms": case_norms, "plans": case_plans, "batch": case_batch,
+CASES = {"refused_set": case_refused_set, "reference_memory": case_reference_memory, "batch_autotune": case_batch_autotune, "thin_pressure": case_thin_pressure, "thin_reference": case_thin_reference, "read_slots": case_read_slots, "small_reads": case_small_reads, "foreign_capture": case_foreign_capture, "read_targets": case_read_targets, "step_graph": case_step_graph, "proxy": case_proxy, "refine_groups": case_refine_groups, "single": case_single, "norms": case_norms, "plans": case_plans, "batch": case_batch,
          "server": case_server, "readback": case_readback, "precision": case_precision,
          "vorticity": case_vorticity, "advection": case_advection}
 

@@ -65,7 +65,8 @@ def test_emulated_case_with_deferred_streams(emu_lib, case):
                                            ("read_slots", False), ("read_slots", True),
                                            ("thin_reference", False), ("thin_pressure", False),
                                            ("batch_autotune", False),
-                                           ("reference_memory", False), ("reference_memory", True)])
+                                           ("reference_memory", False), ("reference_memory", True),
+                                           ("refused_set", False)])
 def test_emulated_host_path(emu_lib, case, deferred):
     """What the host code asks of the runtime (tests/emu/emu_cases.py)."""
     lib, asan = emu_lib
