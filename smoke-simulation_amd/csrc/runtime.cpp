@@ -436,16 +436,21 @@ hipError_t enqueue_refined(smoke_sim* s, long long* launches, long long* sweep_l
 }
 
 // K Jacobi sweeps as launches of plan.sweeps_per_launch fused sweeps each, the
-// remainder in one shorter launch; ping-pongs the two P buffers.
-hipError_t enqueue_jacobi(smoke_sim* s, const smk::JacobiPlan& plan, int sweeps, bool zero_in,
-                          long long* launches)
+// remainder in one shorter launch; ping-pongs the two P buffers.  `fitted`: not
+// a plan that was set; a remainder of one sweep, a whole pass over the fields
+// for it, then shares the last two launches' sweeps (6 sweeps as 5 + 1 / 4 + 2
+// of a 4-sweep plan / 3 + 3: 400x300x350 1446 / 1432 / 1389 us a step, 512^3
+// 4305 / 4270 / 4135).
+hipError_t enqueue_jacobi(smoke_sim* s, const smk::JacobiPlan& plan, bool fitted, int sweeps,
+                          bool zero_in, long long* launches)
 {
     const bool plain = s->prm.jacobi_omega == 1.0;
     // A plane too large for one fused block's 32-bit buffer span: one sweep
     // per launch (same bits).
     const int per_launch = smk::fused_max_zc(s->g.plane) < 1 ? 1 : plan.sweeps_per_launch;
     for (int left = sweeps; left > 0;) {
-        const int t = std::min(left, per_launch);
+        int t = std::min(left, per_launch);
+        if (fitted && per_launch > 1 && left == per_launch + 1) t = (left + 1) / 2;
         const int out = 1 - s->pcur;
         hipError_t e = smk::jacobi_fused(s->g, s->P[s->pcur], s->P[out], s->d, s->flags, plan, t,
                                          (float)s->prm.jacobi_omega, plain ? 1 : 0, zero_in ? 1 : 0,
@@ -528,8 +533,8 @@ hipError_t stage_project(smoke_sim* s, long long* launches)
         }
         if ((e = sweep_mark(s, 0, 0)) != hipSuccess) return e;
         long long sweep_launches = 0;
-        e = enqueue_jacobi(s, s->plan_set ? s->plan : smk::fitted_plan(g, false), p.iterations, zero_in,
-                           &sweep_launches);
+        e = enqueue_jacobi(s, s->plan_set ? s->plan : smk::fitted_plan(g, false), !s->plan_set,
+                           p.iterations, zero_in, &sweep_launches);
         if (e != hipSuccess) return e;
         *launches += sweep_launches;
         if ((e = sweep_mark(s, 1, sweep_launches)) != hipSuccess) return e;
@@ -1425,7 +1430,7 @@ smoke_status smoke_autotune(smoke_sim* s, smoke_jacobi_plan* chosen, double* ms_
                 cand.zc = zc;
                 long long n = 0, n2 = 0;
                 auto run = [&]() {
-                    if (!refined) return enqueue_jacobi(s, cand, K, false, &n);
+                    if (!refined) return enqueue_jacobi(s, cand, false, K, false, &n);
                     s->plan = cand;
                     s->plan_set = true;
                     const hipError_t r = enqueue_refined(s, &n, &n2);

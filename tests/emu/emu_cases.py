@@ -531,6 +531,26 @@ def case_reference_memory():
     g.close()
 
 
+def case_sweep_tail():
+    # A fitted plan leaves no launch for a last sweep alone; a plan that was set
+    # runs as it was set.
+    import ctypes
+    lib = smokesim.load()
+    lib.emu_launches.restype = ctypes.c_longlong
+    for its, given, single in [(6, None, 0), (11, None, 0), (1, None, 1),
+                               (6, dict(sweeps_per_launch=5, tile=0, zc=8), 1)]:
+        sc = scenes.test_scene((14, 12, 10), seed=65, projection=2, iterations=its)
+        g, o = gpu_for(sc), oracle_for(sc, 32)
+        if given:
+            g.set_jacobi_plan(**given)
+        before = lib.emu_launches(b"k_jacobi")
+        assert _sweep_launches(g, sc["dt"]) == -(-its // 5)
+        assert lib.emu_launches(b"k_jacobi") - before == single, (its, given)
+        o.step(sc["dt"], 1)
+        _same_state(g, o, f"{its} sweeps {given}")
+        g.close()
+
+
 def case_refused_set():
     # Without memory for the reference form's own velocity set (after a pressure
     # form) its steps run in place with the same bits; setting the parameters
@@ -634,7 +654,7 @@ def case_foreign_capture():
     g.close()
 
 
-CASES = {"refused_set": case_refused_set, "reference_memory": case_reference_memory, "batch_autotune": case_batch_autotune, "thin_pressure": case_thin_pressure, "thin_reference": case_thin_reference, "read_slots": case_read_slots, "small_reads": case_small_reads, "foreign_capture": case_foreign_capture, "read_targets": case_read_targets, "step_graph": case_step_graph, "proxy": case_proxy, "refine_groups": case_refine_groups, "single": case_single, "norms": case_norms, "plans": case_plans, "batch": case_batch,
+CASES = {"sweep_tail": case_sweep_tail, "refused_set": case_refused_set, "reference_memory": case_reference_memory, "batch_autotune": case_batch_autotune, "thin_pressure": case_thin_pressure, "thin_reference": case_thin_reference, "read_slots": case_read_slots, "small_reads": case_small_reads, "foreign_capture": case_foreign_capture, "read_targets": case_read_targets, "step_graph": case_step_graph, "proxy": case_proxy, "refine_groups": case_refine_groups, "single": case_single, "norms": case_norms, "plans": case_plans, "batch": case_batch,
          "server": case_server, "readback": case_readback, "precision": case_precision,
          "vorticity": case_vorticity, "advection": case_advection}
 

@@ -41,6 +41,7 @@
 #include <functional>
 #include <map>
 #include <memory>
+#include <string>
 #include <thread>
 #include <vector>
 
@@ -83,6 +84,7 @@ namespace {
 std::map<void*, size_t> g_device, g_pinned;  // base and size
 std::map<void*, long long> g_copies;         // by device allocation: copies into it
 long long g_pinned_calls = 0;
+std::map<std::string, long long> g_launches;  // by kernel
 size_t g_refuse_above = SIZE_MAX;  // larger allocations are refused
 std::recursive_mutex g_mu;                   // held by the calls several threads make
 using Lock = std::lock_guard<std::recursive_mutex>;
@@ -325,6 +327,7 @@ hipError_t emu_last_error() { return hipSuccess; }
 void emu_launch(const char* name, std::function<void()> fn, dim3 grid, dim3 block, hipStream_t st)
 {
     check(st);
+    g_launches[name] += 1;
     if (st && st->capturing) {
         st->rec.push_back([=]() { run(name, fn, grid, block); });
         return;
@@ -563,7 +566,7 @@ hipError_t hipEventElapsedTime(float* ms, hipEvent_t a, hipEvent_t b)
     return hipSuccess;
 }
 
-// What a test asks of the emulator: pinned allocations asked for so far and
+// What a test asks of the emulator: launches of a kernel, pinned allocations asked for so far and
 // held now, the device bytes held, the asynchronous copies into the device
 // allocation at `base`; and to refuse allocations of more than n bytes.
 long long emu_pinned_calls() { return g_pinned_calls; }
@@ -574,6 +577,7 @@ long long emu_device_bytes()
     for (const auto& a : g_device) n += (long long)a.second;
     return n;
 }
+long long emu_launches(const char* kernel) { return g_launches[kernel]; }
 void emu_refuse_above(size_t n) { g_refuse_above = n; }
 long long emu_copies_into(void* base)
 {

@@ -66,7 +66,7 @@ def test_emulated_case_with_deferred_streams(emu_lib, case):
                                            ("thin_reference", False), ("thin_pressure", False),
                                            ("batch_autotune", False),
                                            ("reference_memory", False), ("reference_memory", True),
-                                           ("refused_set", False)])
+                                           ("refused_set", False), ("sweep_tail", False)])
 def test_emulated_host_path(emu_lib, case, deferred):
     """What the host code asks of the runtime (tests/emu/emu_cases.py)."""
     lib, asan = emu_lib
