@@ -832,19 +832,22 @@ bool pageable(const void* p)
 // pinned slots, one per thread (a thread for every 1 MB, at most 8), so that
 // DMA, memcpy and page faults of different pieces overlap: 2.0 ms.
 //
-// Reads below 4 MB take the runtime's copy: with slots they were no faster
-// where a wait for the GPU takes a few us (ms, runtime's / slots: 1 MB 0.08 /
-// 0.08, 2 MB 0.13 / 0.13, 4 MB 0.24 / 0.22, 5 MB 0.30 / 0.26, 8 MB 0.47 /
-// 0.38), and every piece is one more wait where it takes 0.1 ms (64 KB 0.03 /
-// 0.13, 1 MB 0.15 / 0.28, 2 MB 0.29 / 0.45, 3.5 MB 0.58 / 0.64).
-constexpr size_t kSlotReadBytes = 4u << 20;
+// Below 4 MB the slots take the whole read in one copy, with one wait, and this
+// thread copies it out in pieces of 512 KB (from 1 MB on a single memcpy goes
+// past the caches, slower into new pages): a wait for the GPU may take 0.1 ms,
+// so a wait for every piece cost more than the overlap gave.  us, runtime's copy
+// / a wait a piece / this, into touched pages: 256 KB 34 / 41 / 33, 1 MB 78 / 76
+// / 66, 2 MB 130 / 147 / 115, 3.9 MB 250 / 205 / 195; into new ones: 77 / 84 /
+// 76, 303 / 250 / 247, 540 / 490 / 465, 1085 / 850 / 885.
+constexpr size_t kMinSlotRead = 64u << 10, kThreadedRead = 4u << 20;
+static_assert(kThreadedRead <= kReadSlots * kReadSlotBytes, "the slots take it whole");
 smoke_status copy_to_host(smoke_sim* s, void* dst, const void* dev, size_t bytes)
 {
     ReadSlots* const slots = read_slots(s->device);
     std::unique_lock<std::mutex> lk;
     if (slots) lk = std::unique_lock<std::mutex>(slots->mu, std::defer_lock);
     int device = -1;
-    if (bytes < kSlotReadBytes || !pageable(dst) || hipGetDevice(&device) != hipSuccess ||
+    if (bytes < kMinSlotRead || !pageable(dst) || hipGetDevice(&device) != hipSuccess ||
         device != s->device || !slots || !lk.try_lock() || !slots_ready(*slots, bytes)) {
         if (lk.owns_lock()) lk.unlock();
         HIP_TRY(hipMemcpyAsync(dst, dev, bytes, hipMemcpyDeviceToHost, s->stream));
@@ -853,6 +856,14 @@ smoke_status copy_to_host(smoke_sim* s, void* dst, const void* dev, size_t bytes
     }
     char* const out = static_cast<char*>(dst);
     const char* const in = static_cast<const char*>(dev);
+    if (bytes < kThreadedRead) {
+        HIP_TRY(hipMemcpyAsync(slots->mem, in, bytes, hipMemcpyDeviceToHost, s->stream));
+        HIP_TRY(hipStreamSynchronize(s->stream));
+        constexpr size_t kPiece = 512u << 10;
+        for (size_t at = 0; at < bytes; at += kPiece)
+            std::memcpy(out + at, slots->mem + at, std::min(kPiece, bytes - at));
+        return SMOKE_OK;
+    }
     const int threads = (int)std::min<size_t>(kReadSlots, bytes >> 20);
     const size_t width = std::min(kReadSlotBytes, (bytes / threads + 4095) / 4096 * 4096);
     std::atomic<int> failed{(int)hipSuccess};

@@ -370,14 +370,24 @@ def _emu(name, *args):
 
 
 def case_small_reads():
-    # Reads below 4 MB are the runtime's copies: no pinned pieces.
+    # Reads that come to less than the pinned slots' size are the runtime's
+    # copies; from then on a small read is one copy into the slots.
     rng = np.random.default_rng(12)
-    for dims in ((40, 33, 30), (101, 100, 99)):  # 155 KB, 3.8 MB
+    for dims, n in (((40, 33, 30), 20), ((101, 100, 99), 3)):  # 155 KB, 3.8 MB
         x = rng.standard_normal(dims[::-1]).astype(np.float32)
         with smokesim.Simulation(*dims, density=x) as g:
-            for _ in range(6):
+            for _ in range(n):
                 same_bits(g.get_density(0), x, f"{dims}")
     assert _emu("emu_pinned_calls") == 0
+    with smokesim.Simulation(101, 100, 99, density=x) as g:
+        for _ in range(6):
+            same_bits(g.get_density(0), x, "with slots")
+        assert _emu("emu_pinned_calls") == 1 == _emu("emu_pinned_held")
+        for dims in ((20, 17, 13), (40, 33, 30), (64, 64, 33)):
+            y = rng.standard_normal(dims[::-1]).astype(np.float32)
+            with smokesim.Simulation(*dims, density=y) as h:
+                same_bits(h.get_density(0), y, f"with slots {dims}")
+    assert _emu("emu_pinned_held") == 0
 
 
 def case_read_slots():

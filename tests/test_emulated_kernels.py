@@ -61,7 +61,7 @@ def test_emulated_case_with_deferred_streams(emu_lib, case):
 
 
 @pytest.mark.parametrize("case,deferred", [("read_targets", False), ("read_targets", True),
-                                           ("foreign_capture", False), ("small_reads", False),
+                                           ("foreign_capture", False), ("small_reads", False), ("small_reads", True),
                                            ("read_slots", False), ("read_slots", True),
                                            ("thin_reference", False), ("thin_pressure", False),
                                            ("batch_autotune", False),

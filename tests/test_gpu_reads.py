@@ -10,8 +10,9 @@ import smokesim
 
 pytestmark = pytest.mark.gpu
 
-# 56 KB and just below 4 MB; just above, where pinned slots of 2 MB begin (four
-# threads), all eight threads with pieces of under 2 MB, and several each
+# 56 KB and just below 4 MB (once the pinned slots are there, one copy into them);
+# just above, where a thread takes each 2 MB slot (four of them), all eight with
+# pieces of under 2 MB, and several pieces each
 DIMS = [(29, 23, 21), (128, 128, 63), (128, 128, 65), (160, 151, 149), (187, 165, 160)]
 
 
@@ -42,9 +43,11 @@ class Memory:
 @pytest.mark.parametrize("kind", ["pinned", "device"])
 def test_read_targets(dims, kind):
     x = np.random.default_rng(3).standard_normal(dims[::-1]).astype(np.float32)
-    with smokesim.Simulation(*dims, density=x) as g:
+    with smokesim.Simulation(*dims, density=x) as g, smokesim.Simulation(187, 165, 160) as other:
         for _ in range(3):
             assert np.array_equal(g.get_density(0), x)
+        other.get_density(0)  # 19 MB: the slots are there now
+        assert np.array_equal(g.get_density(0), x)
         m = Memory(kind, x.nbytes)
         smokesim._check(g.lib.smoke_get_density(g.h, 0, ctypes.cast(m.p, ctypes.POINTER(ctypes.c_float))))
         assert np.array_equal(m.floats(), x.ravel())
