@@ -14,12 +14,13 @@
 // Grids of at most one box per CU (k_ref_faces_box): the launch is a chain of
 // latencies, and a box in LDS with all CUs busy is the shortest one.  80^3:
 // 13.3 us per launch of 4 half-sweeps (2.3 the launch itself, 5 the loads and
-// stores, 1.4 each half-sweep), 4 x 4.6 us one by one, 16.4 us marched.
+// stores, 1.4 each half-sweep), 4 x 4.5 us one by one, 19.3 us marched.
 // Larger grids (k_ref_faces_march): a column marched up z re-reads far less
-// halo.  256x240x248, 5 half-sweeps per launch: 133 us against 5 x 85 us; boxes
-// 306 us per 4.  150x96x121, 4 per launch: 24 us against 4 x 11.2 us (boxes 42
-// per 4): there FP64 conversions and VALU issue bind (2 % of the cells next to
-// a solid), memory at 256.
+// halo.  Empty 256x240x248, 5 half-sweeps per launch: 127 us against 5 x 80 us;
+// boxes 306 us per 4.  150x96x121, 4 per launch: 21.5 us against 4 x 10.5 us (boxes
+// 42 per 4): there FP64 conversions and VALU issue bind, memory at 256.  Cells next
+// to a solid take longer (256^3, 5 a launch: 138 us empty, 141 with 5 % solid boxes).
+// Grids thin in x or y keep one half-sweep per launch (reference_in_place).
 #pragma once
 
 #include "step_device.h"
@@ -348,10 +349,10 @@ __global__ __launch_bounds__(TP * TY) void k_ref_faces_march(
 // one barrier per plane.  The pairs are skewed as above; a cell needs only its
 // neighbours' pressures, so exactly H cells go stale on every side.
 //
-// us per half-sweep, one per launch before: 113x90x101 6.3 -> 3.2, 80^3 4.5 ->
-// 2.6, 256x240x248 44 -> 11.8.  Small grids are a chain of LDS latencies and
+// us per half-sweep, one per launch -> here: 113x90x101 6.1 -> 3.2, 80^3 4.1 ->
+// 2.5, 256x240x248 51 -> 11.6.  Small grids are a chain of LDS latencies and
 // barriers (16-pair columns of half the threads then beat 32-pair ones: 48x40x57
-// 2.1 against 2.7), large ones 3.5 TB/s of loads and stores over VALU issue.
+// 1.9 against 2.5), large ones 3.5 TB/s of loads and stores over VALU issue.
 template <int TP, int TY, int H>
 struct PressureColumn {
     static_assert(H % 2 == 0 && 64 % TP == 0, "whole pairs, whole rows per wave");

@@ -715,9 +715,10 @@ hipError_t project_reference_half(const Grid& g, float* u, float* v, float* w,
 // (redblack.h has both sides).  Else columns, 4 half-sweeps per launch, or where
 // the two sets of faces and the flags approach the 256 MB memory-side cache (a
 // launch is then bound by memory and fewer passes pay for the larger halo) the
-// better fitting of 5 and 6.  us per half-sweep with 4 / 5 / 6: 160^3 (125 MB)
-// 8.6 / 10.0 / 9.5, 192x180x188 (191 MB) 11.6 / 11.9 / 11.7, 224x200x210 (271 MB)
-// 19.7 / 16.9 / 16.0, 256x240x248 29.4 / 26.6 / 29.0 (one column more for 6).
+// better fitting of 5 and 6.  us per half-sweep of empty grids with 4 / 5 / 6:
+// 160^3 (125 MB) 7.8 / 9.0 / 8.7, 192x180x188 (191 MB) 10.7 / 11.0 / 10.6,
+// 224x200x210 (271 MB) 19.5 / 15.7 / 14.4, 256x240x248 29.0 / 25.5 / 26.7 (one
+// column more for 6).
 constexpr int kBoxX = 24, kBoxY = 10, kBoxZ = 10;
 struct FacesRoute {
     bool boxed;
@@ -922,9 +923,9 @@ hipError_t jacobi_fused(const Grid& g, const float* pin, float* pout, const floa
 
 // 4 or 6 half-sweeps per launch, whichever takes fewer steps per half-sweep;
 // narrow columns where the grid is too small to fill the CUs with wide ones.
-// us per half-sweep, narrow 4 / 4 / 6: 48x40x57 2.1 / 2.8 / 2.7, 80^3 2.6 / 2.9
-// / 2.8, 113x90x101 3.2 / 3.3 / 3.4, 150^3 4.8 / 5.0 / 4.7, 256x240x248 13.3 /
-// 12.3 / 11.8.
+// us per half-sweep, narrow 4 / 4 / 6: 48x40x57 1.9 / 2.5 / 2.5, 80^3 2.5 / 2.8
+// / 2.7, 113x90x101 3.2 / 3.2 / 3.3, 150^3 6.0 / 4.8 / 4.5, 256x240x248 19.2 /
+// 11.8 / 11.6.
 struct PressureRoute {
     bool narrow;
     int H;
