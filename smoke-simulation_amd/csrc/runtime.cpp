@@ -6,6 +6,7 @@
 // step is a fixed sequence of kernel launches on that stream; nothing in it
 // allocates or synchronises unless the caller asks for the density back.
 #include <hip/hip_runtime.h>
+#include <pthread.h>
 
 #include <algorithm>
 #include <atomic>
@@ -14,10 +15,8 @@
 #include <cstdio>
 #include <cstring>
 #include <deque>
-#include <exception>
 #include <mutex>
 #include <string>
-#include <thread>
 #include <vector>
 
 #include "sim_state.h"
@@ -879,17 +878,35 @@ smoke_status copy_to_host(smoke_sim* s, void* dst, const void* dev, size_t bytes
         }
         if (e != hipSuccess) failed = (int)e;
     };
-    std::vector<std::thread> helpers;
-    try {
-        helpers.reserve((size_t)threads);
-        for (int k = 1; k < threads; ++k) helpers.emplace_back(run, k, true);
-    } catch (const std::exception&) {
-        // The pieces of a thread that could not start are copied below.
+    // Threads with small stacks, which the C library keeps for the next read
+    // (of 8 MB ones it keeps five, and gives back and sets up the others' thread
+    // data in the caller's heap each time: the caller's own freed memory then went
+    // back to the system and was faulted in again).
+    using Run = decltype(run);
+    struct Helper {
+        Run* run;
+        int slot;
+        pthread_t id;
+    } helpers[kReadSlots];
+    const auto enter = [](void* h) -> void* {
+        (*static_cast<Helper*>(h)->run)(static_cast<Helper*>(h)->slot, true);
+        return nullptr;
+    };
+    pthread_attr_t small;
+    const bool able = pthread_attr_init(&small) == 0;
+    int started = 1;
+    if (able) {
+        (void)pthread_attr_setstacksize(&small, 2u << 20);
+        for (; started < threads; ++started) {
+            helpers[started].run = &run;
+            helpers[started].slot = started;
+            if (pthread_create(&helpers[started].id, &small, enter, &helpers[started]) != 0) break;
+        }
+        (void)pthread_attr_destroy(&small);
     }
-    const int started = (int)helpers.size() + 1;
     run(0, false);
-    for (int k = started; k < threads; ++k) run(k, false);
-    for (std::thread& t : helpers) t.join();
+    for (int k = started; k < threads; ++k) run(k, false);  // of those that could not start
+    for (int k = 1; k < started; ++k) (void)pthread_join(helpers[k].id, nullptr);
     const hipError_t done = hipStreamSynchronize(s->stream);  // no copy still writes a slot
     HIP_TRY((hipError_t)failed.load());
     HIP_TRY(done);
