@@ -414,8 +414,9 @@ smoke_status smoke_batch_synchronize(smoke_batch* batch);
 smoke_status smoke_batch_set_jacobi_plan(smoke_batch* batch, const smoke_jacobi_plan* plan);
 smoke_status smoke_batch_get_jacobi_plan(const smoke_batch* batch, smoke_jacobi_plan* out);
 /* Autotuner of the batched sweep sequence (the plan in force, then 2..6 sweeps
- * per launch x the four tiles x z-chunks of 8, 16, 32, 64, 128 and 256 planes);
- * invalidates a captured graph. */
+ * per launch x the four tiles x z-chunks of 32, 64, 128 and 256 planes, and of 8
+ * and 16 for batches that leave compute units idle with 32); invalidates a
+ * captured graph. */
 smoke_status smoke_batch_autotune(smoke_batch* batch, smoke_jacobi_plan* chosen, double* ms_per_sweep);
 /* Step latencies (ms, HIP events around each step on the batch's stream) of
  * the last `cap` steps, oldest first. */

@@ -620,8 +620,20 @@ smoke_status smoke_batch_autotune(smoke_batch* b, smoke_jacobi_plan* chosen, dou
     double best_ms = -1.0;
     const int tiles[4] = {smk::JacobiPlan::TILE_32x32, smk::JacobiPlan::TILE_64x16,
                           smk::JacobiPlan::TILE_64x32, smk::JacobiPlan::TILE_32x64};
-    // Short chunks too: a small batch occupies few CUs with long ones.
+    // Short chunks too, where those of 32 planes leave CUs without a workgroup
+    // (elsewhere they only add planes to march and time to the search: 64 volumes
+    // of 32..160 a side 2.4 s instead of 1.6).
     const int zcs[6] = {8, 16, 32, 64, 128, 256};
+    auto idle_cus = [&](int t, int tile) {
+        smk::JacobiPlan p;
+        p.sweeps_per_launch = t;
+        p.tile = tile;
+        p.zc = std::min(32, b->zc_cap);
+        smk::StageTable tab;
+        int total = 0;
+        fill_table(tab, b->sims, kTabJacobi, p, &total);
+        return total < b->cus;
+    };
     hipError_t e = hipSuccess;
     auto time = [&](int t, int tile, int zc) {
         b->plan.sweeps_per_launch = t;
@@ -646,9 +658,11 @@ smoke_status smoke_batch_autotune(smoke_batch* b, smoke_jacobi_plan* chosen, dou
     // The plan in force (fitted or given) first: another has to be faster.
     time(given.sweeps_per_launch, given.tile, given.zc);
     for (int t = 2; t <= 6 && e == hipSuccess; ++t)
-        for (int tile : tiles)
+        for (int tile : tiles) {
+            const bool idle = idle_cus(t, tile);
             for (int zc : zcs)
-                if (e == hipSuccess) time(t, tile, zc);  // a failed candidate ends the search
+                if (e == hipSuccess && (idle || zc >= 32)) time(t, tile, zc);  // a failed one ends the search
+        }
     (void)hipEventDestroy(ev[0]);
     (void)hipEventDestroy(ev[1]);
     b->plan = b->reported = best;
